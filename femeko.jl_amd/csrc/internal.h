@@ -287,6 +287,10 @@ struct fk_mesh {
     int nblocks = 0;                  // persistent grid of the solver kernels
     int64_t chunk = 0;                // rows per logical block
 
+    // register-resident PCG (resident.hip): all-reduce slots, exchanged row values
+    fk::DevBuf<unsigned long long> res_slots;
+    fk::DevBuf<double> res_w;
+
     fk::PcgWork<double> w64;
     fk::PcgWork<float> w32;
 };
@@ -331,6 +335,8 @@ inline void values_changed(fk_mesh *m) {
     m->sell64_valid = false;
     m->sell32_valid = false;
 }
+// FP64 PCG in one cooperative launch (resident.hip); false: not for this mesh
+bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, CgState *out);
 CgState run_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref);
 int solve_f32_increment(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, int64_t *iters);
 int solve_f32_free(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, double bb_ref,

@@ -1640,6 +1640,10 @@ static CgState run_pcg(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref)
     PcgWork<T> &w = work<T>(m);
     const int nb = m->nblocks;
     sync_solver_values<T>(m);
+    if constexpr (sizeof(T) == 8) {
+        CgState done{};
+        if (resident_pcg_f64(m, rtol, max_iter, bb_ref, &done)) return done;
+    }
     k_cg_init<T><<<nb, kBlock, 0, st>>>(w.x.get(), w.r.get(), w.p.get(), w.dinv.get(), w.part_rz.get(),
                                         w.part_bb.get(), m->nv, m->chunk, nb);
     k_cg_start<<<1, kBlock, 0, st>>>(w.part_bb.get(), nb, bb_ref, rtol, max_iter, w.state.get());

@@ -1,0 +1,140 @@
+"""The register-resident PCG (one cooperative launch per solve on the stencil
+copy) against the three-kernel iteration, which a context with timing enabled
+runs: row counts at the edges of its launch shapes, elongated grids whose
+windows merge or split, odd tails, iteration limit and breakdown.
+
+Bars: both solves stop at ||r|| < 1e-12 ||b||, so their potentials agree to
+the suite's 1e-9; iteration counts agree to 5% + 4 (rounding moves the
+iteration at which a slowly falling residual crosses the tolerance)."""
+import numpy as np
+import pytest
+
+from femeko_hip import FemekoHIPError
+from femeko_hip import workloads as W
+from femeko_hip.device import Context, DeviceMesh
+from femeko_hip.mesh import MESH, MU0, _kuhn_local_offsets, element_volumes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def contexts():
+    plain, timed = Context(0), Context(0)
+    timed.set_timing(True)
+    yield plain, timed
+    plain.close()
+    timed.close()
+
+
+def _box(nx, ny, nz):
+    """Kuhn mesh of nx x ny x nz unit cells, x fastest."""
+    m, l = nx + 1, ny + 1
+    K, J, I = np.meshgrid(np.arange(nz + 1), np.arange(l), np.arange(m), indexing="ij")
+    p = np.asfortranarray(np.stack([I.ravel(), J.ravel(), K.ravel()]).astype(float))
+    ck, cj, ci = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    base = (ci + m * (cj + l * ck)).ravel()
+    off = _kuhn_local_offsets()
+    t = base[:, None, None] + (off[:, :, 0] + m * (off[:, :, 1] + l * off[:, :, 2]))[None]
+    t = np.asfortranarray((t.reshape(-1, 4).T + 1).astype(np.int32))
+    return MESH(p=p, t=t, VE=element_volumes(p, t))
+
+
+def _both(contexts, mesh, mu, mask, g, precision="f64", rtol=1e-12, fmt=None):
+    out = []
+    for ctx in contexts:
+        dm = DeviceMesh(mesh, ctx)
+        try:
+            dm.set_coefficient(mu)
+            dm.assemble()
+            dm.set_dirichlet(mask, g)
+            rep = dm.solve(precision, rtol=rtol)
+            assert fmt is None or dm.solver_format()[0] == fmt
+            first = dm.potential()
+            again = dm.solve(precision, rtol=rtol)
+            assert np.array_equal(first, dm.potential()) and again.iterations == rep.iterations
+            out.append((first, rep))
+        finally:
+            dm.close()
+    (a, ra), (b, rb) = out
+    assert ra.relres < rtol and rb.relres < rtol
+    assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
+    assert abs(ra.iterations - rb.iterations) <= 4 + rb.iterations // 20
+
+
+# 27 rows; 512 rows exactly; one more plane; the last n of each launch shape
+# and the first of the next (rows (n + 1)^3 against 256 x 512, 1024, ... 4096)
+@pytest.mark.parametrize("n", [2, 7, 8, 19, 49, 50, 63, 64, 72, 73, 79, 80, 85, 86, 90, 91, 95, 96, 100, 101])
+def test_launch_shapes(contexts, n):
+    pr = W.linear(n)
+    _both(contexts, pr.mesh, pr.mu, pr.mask, pr.g, fmt="stencil")
+
+
+# one cell thick (too much padding for the stencil copy: SELL), long columns,
+# flat plates: one merged window, split windows, and offsets too far apart for
+# three windows (the three-kernel iteration on both)
+@pytest.mark.parametrize("dims", [(1, 1, 200), (3, 5, 41), (200, 3, 3), (90, 90, 2), (2, 90, 90), (700, 20, 3)])
+def test_elongated_grids(contexts, dims):
+    mesh = _box(*dims)
+    rng = np.random.default_rng(3)
+    mu = MU0 * rng.uniform(1.0, 50.0, mesh.nt)
+    top = np.array(dims, float)[:, None]
+    mask = ((mesh.p == 0.0) | (mesh.p == top)).any(axis=0)
+    inner = rng.random(mesh.nv) < 0.5     # a one-cell box has no interior: free half of its nodes
+    mask = mask & ~inner if not (~mask).any() else mask
+    g = np.where(mask, rng.normal(size=mesh.nv), 0.0)
+    _both(contexts, mesh, mu, mask.astype(np.uint8), g)
+
+
+def test_limit_and_breakdown(contexts):
+    pr = W.linear(20)
+    dm = DeviceMesh(pr.mesh, contexts[0])
+    try:
+        dm.set_coefficient(pr.mu)
+        dm.assemble()
+        dm.set_dirichlet(pr.mask, pr.g)
+        rep = dm.solve("f64", rtol=1e-12, max_iter=7, raise_on_error=False)
+        assert rep.status == 6 and rep.iterations == 7
+        assert dm.solve("f64", rtol=1e-10).relres < 1e-10
+        # zero Dirichlet data: b = 0, nothing to iterate
+        dm.set_dirichlet(pr.mask, np.zeros_like(pr.g))
+        assert dm.solve("f64", rtol=1e-10).iterations == 0 and not dm.potential().any()
+        # indefinite coefficients that keep every diagonal positive break down or diverge with a status
+        mu = pr.mu.copy()
+        mu[::7] *= -2.0
+        dm.set_coefficient(mu)
+        dm.assemble()
+        dm.set_dirichlet(pr.mask, pr.g)
+        with pytest.raises(FemekoHIPError):
+            dm.solve("f64", rtol=1e-12, max_iter=300)
+    finally:
+        dm.close()
+
+
+def test_two_contexts_in_two_threads():
+    import threading
+
+    probs = [W.linear(40), W.linear(56)]
+    ref, got, ctxs, dms = [], [[], []], [Context(0), Context(0)], []
+    for pr, ctx in zip(probs, ctxs):
+        dm = DeviceMesh(pr.mesh, ctx)
+        dm.set_coefficient(pr.mu)
+        dm.assemble()
+        dm.set_dirichlet(pr.mask, pr.g)
+        dm.solve("f64", rtol=1e-10)
+        ref.append(dm.potential())
+        dms.append(dm)
+
+    def work(k):
+        for _ in range(6):
+            dms[k].solve("f64", rtol=1e-10)
+            got[k].append(dms[k].potential())
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for k in range(2):
+        dms[k].close()
+        ctxs[k].close()
+        assert len(got[k]) == 6 and all(np.array_equal(ref[k], u) for u in got[k])
