@@ -337,6 +337,9 @@ inline void values_changed(fk_mesh *m) {
 }
 // FP64 PCG in one cooperative launch (resident.hip); false: not for this mesh
 bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, CgState *out);
+// the same for the FP32 recursion with FP64 residual replacement
+bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
+                      int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status);
 CgState run_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref);
 int solve_f32_increment(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, int64_t *iters);
 int solve_f32_free(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, double bb_ref,

@@ -57,6 +57,15 @@ struct ResidentArgs {
     int32_t wrow[kResWindows];    // row - i0 of an element - its LDS index, by window
     double bb_ref, rtol;
     int64_t max_iter;
+    // residual replacement (FP32 recursion, FP64 solution u)
+    double *u;                    // FP64 solution, accumulates x / s
+    const double *b;              // right-hand side, null: 0
+    double *r64;                  // FP64 residual
+    const double *val64, *diag64;
+    T *p;                         // the direction of the own rows over a replacement
+    RuState *ru;
+    double s, target2, thresh64, delta2;
+    int32_t G;                    // iterations between two checks of the drop
 };
 
 // A copy of v that the compiler takes for a new value: addresses computed from
@@ -67,7 +76,12 @@ __device__ __forceinline__ int32_t fresh(int32_t v) {
     return v;
 }
 
-// row of window element li (LDS index)
+// LDS index of the e-th window element (the windows in LDS order, the own rows
+// left out; elements past the last share one spare slot) and its row (spare: none)
+template <typename T>
+__device__ __forceinline__ int32_t window_lds(const ResidentArgs<T> &A, int32_t R, int32_t e) {
+    return min(e < A.lown ? e : e + R, A.wbeg[kResWindows]);
+}
 template <typename T>
 __device__ __forceinline__ int32_t window_row(const ResidentArgs<T> &A, int32_t i0, int32_t li) {
     int32_t d = A.wrow[0];
@@ -76,172 +90,327 @@ __device__ __forceinline__ int32_t window_row(const ResidentArgs<T> &A, int32_t 
     return li < A.wbeg[kResWindows] ? i0 + li + d : -1;
 }
 
+template <typename T>
+constexpr bool x_in_lds(int rpt) {
+    return sizeof(T) == 8 && rpt >= 4;
+}
+
+constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursion gives up
+
 // RPT rows per thread, the values of the first NK of them in registers (the
 // others are streamed from L2 / MALL, a row ahead of their use); U window
 // elements per thread at most.
-template <typename T, int BLOCK, int RPT, int NK, int U>
+//
+// REFINE (T = float): the reliable updates of solve.hip inside the launch. At
+// the end of every G iterations in which ||r||^2 has fallen by delta2 since
+// the last replacement, and when the recursion has reached its target, x / s
+// is folded into the FP64 solution u, the FP64 residual b - A u of the free
+// rows replaces the recursion's (times s), and p is kept; a recursion that has
+// drifted below the true residual, or broken down, restarts from p = z. The
+// solve ends on the FP64 residual.
+template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE>
 __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A) {
     extern __shared__ char lds_raw[];
     T *win = reinterpret_cast<T *>(lds_raw);
-    __shared__ double sh[5 * (BLOCK / 64 + 1) + 1];
+    __shared__ double sh[kReduceShared];
     constexpr int K = kResK, R = BLOCK * RPT;
+    // x of the FP64 shapes with many rows per thread waits in LDS, past the windows
+    constexpr bool XLDS = x_in_lds<T>(RPT);
+    T *xs = win + A.wbeg[kResWindows] + 1;
+    constexpr bool AHEAD = RPT > 1 && (sizeof(T) == 4 || RPT <= 3);
     const int32_t i0 = logical_block(A.nb) * R;
     const int32_t tid = threadIdx.x;
     const AgentRows<T> rows(A.w, A.stride);
     const ValueColumns<T> vals(A.val, A.K, A.ld);
     const int32_t n = A.n;
-    uint32_t tag = 0;
-    if (tid == 0) sh[5 * (BLOCK / 64 + 1)] = 0.0;
+    uint32_t tag = 1;
+    if (tid == 0) sh[kReduceShared - 1] = 0.0;
 
-    T d[RPT], g[RPT], x[RPT], z[RPT], p[RPT], w[RPT];
-    T zw[U];
-    int32_t li[U];  // LDS index of this thread's window elements (one spare element past the windows)
-    T vf[NK > 0 ? NK : 1][K], vb[NK > 0 ? NK : 1][K];
-#pragma unroll
+    // z = D^-1 r of the own rows goes out
+    double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
     for (int j = 0; j < RPT; ++j) {
         const int32_t row = i0 + j * BLOCK + tid;
-        const bool in = row < n;
-        d[j] = in ? A.dinv[row] : T(0);
-        const bool free = d[j] != T(0);
-        g[j] = free ? T(1) / d[j] : T(0);
-        x[j] = T(0);
-        z[j] = free ? d[j] * A.r0[row] : T(0);
-        p[j] = z[j];
-        if (in) rows.store(1, row, z[j]);
-        win[A.lown + j * BLOCK + tid] = p[j];
+        if (row >= n) continue;
+        const T dj = A.dinv[row];
+        T r = T(0);
+        if (dj != T(0)) r = REFINE ? static_cast<T>(A.s * A.r64[row]) : A.r0[row];
+        rows.store(tag, row, dj * r);
     }
-#pragma unroll
-    for (int j = 0; j < NK; ++j)
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            vf[j][k] = vb[j][k] = T(0);
-            if (k < A.K) {
-                vf[j][k] = vals.load(k, i0 + j * BLOCK + tid);
-                vb[j][k] = vals.load(k, i0 + j * BLOCK + tid - A.off[k]);
-            }
-        }
-    double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    bool alive = all_reduce5<BLOCK>(s, A.slots, A.nb, ++tag, sh);  // every z is out
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        // the windows' elements in LDS order, the own rows left out
-        const int32_t e = tid + u * BLOCK;
-        li[u] = min(e < A.lown ? e : e + R, A.wbeg[kResWindows]);
-        zw[u] = rows.load(1, window_row(A, i0, li[u]));
-        win[li[u]] = zw[u];
-    }
-    __syncthreads();
+    bool alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
 
     double rr = 0.0, thresh = 0.0, bb = A.bb_ref;
     int64_t it = 0;
     int code = alive ? -1 : FK_ERR_HIP;  // -1: running
+    [[maybe_unused]] double rr64 = 0.0, rr_last = 1.0;
+    [[maybe_unused]] int32_t nrep = 0, restarts = 0, until_check = A.G;
+    bool restart = true;  // p = z
     while (code < 0) {
-        ++tag;
-        // q = A p in difference form; w = D^-1 q
-#pragma unroll
-        for (int k = 0; k < 5; ++k) s[k] = 0.0;
-        T sf[K], sb[K];
-        [[maybe_unused]] const int32_t t0 = fresh(tid);
-        if constexpr (NK < RPT) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                sf[k] = sb[k] = T(0);
-                if (k < A.K) {
-                    sf[k] = vals.load(k, i0 + NK * BLOCK + t0);
-                    sb[k] = vals.load(k, i0 + NK * BLOCK + t0 - A.off[k]);
-                }
-            }
-        }
+        // ---- a run of iterations from z (exchanged) and p: state into registers
+        const int32_t tl = fresh(tid);
+        T d[RPT], g[RPT], x[XLDS ? 1 : RPT], z[RPT], p[RPT], w[RPT];
+        T zw[U];
+        T vf[NK > 0 ? NK : 1][K], vb[NK > 0 ? NK : 1][K];
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
-            const int32_t l = j * BLOCK + fresh(tid), row = i0 + l;
-            T a0 = T(0), a1 = T(0);
-            if (j < NK) {
-                const int jk = j < NK ? j : 0;
+            const int32_t row = i0 + j * BLOCK + tl, at = min(row, n - 1);
+            const T dj = A.dinv[at], pj = restart ? T(0) : A.p[at];
+            z[j] = rows.load(tag, row);  // 0 past the last row
+            d[j] = row < n ? dj : T(0);
+            p[j] = restart || row >= n ? z[j] : pj;
+            if (XLDS)
+                xs[j * BLOCK + tl] = T(0);
+            else
+                (XLDS ? xs[j * BLOCK + tl] : x[XLDS ? 0 : j]) = T(0);
+            if (restart) win[A.lown + j * BLOCK + tl] = p[j];
+        }
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) g[j] = d[j] != T(0) ? T(1) / d[j] : T(0);
+#pragma unroll
+        for (int j = 0; j < NK; ++j)
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                vf[j][k] = vb[j][k] = T(0);
+                if (k < A.K) {
+                    vf[j][k] = vals.load(k, i0 + j * BLOCK + tl);
+                    vb[j][k] = vals.load(k, i0 + j * BLOCK + tl - A.off[k]);
+                }
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int32_t li = window_lds(A, R, tl + u * BLOCK);
+            zw[u] = rows.load(tag, window_row(A, i0, li));
+            if (restart) win[li] = zw[u];
+        }
+        __syncthreads();
+        [[maybe_unused]] bool moved = false;  // an iteration done in this run
+        [[maybe_unused]] int act = 0;         // why it ended: 1 replace r, 2 drop x and restart
+        while (true) {
+            ++tag;
+            // q = A p in difference form; w = D^-1 q
+#pragma unroll
+            for (int k = 0; k < 5; ++k) s[k] = 0.0;
+            T sf[K], sb[K];
+            [[maybe_unused]] const int32_t t0 = fresh(tid);
+            if constexpr (NK < RPT) {
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    a0 += vf[jk][k] * (win[A.lf[k] + l] - p[j]);
-                    a1 += vb[jk][k] * (win[A.lb[k] + l] - p[j]);
+                    sf[k] = sb[k] = T(0);
+                    if (k < A.K) {
+                        sf[k] = vals.load(k, i0 + NK * BLOCK + t0);
+                        sb[k] = vals.load(k, i0 + NK * BLOCK + t0 - A.off[k]);
+                    }
                 }
-            } else {
-                T nf[K], nbk[K];
-                if (j + 1 < RPT) {
+            }
+            // the neighbours of a row are loaded together, and where registers
+            // allow a row ahead: one LDS latency per row, not one per neighbour
+            T pf[K], pb[K];
+            const auto neighbours = [&](int j, T(&f)[K], T(&b)[K]) {
+                const int32_t l = j * BLOCK + fresh(tid);
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    f[k] = win[A.lf[k] + l];
+                    b[k] = win[A.lb[k] + l];
+                }
+            };
+            if constexpr (AHEAD) neighbours(0, pf, pb);
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                const int32_t row = i0 + j * BLOCK + fresh(tid);
+                T nf[K], nbk[K], nv[K], nvb[K];
+                if (AHEAD && j + 1 < RPT) neighbours(j + 1, nf, nbk);
+                if (!AHEAD) neighbours(j, pf, pb);
+                if (NK < RPT && j >= NK && j + 1 < RPT) {
 #pragma unroll
                     for (int k = 0; k < K; ++k) {
-                        nf[k] = nbk[k] = T(0);
+                        nv[k] = nvb[k] = T(0);
                         if (k < A.K) {
-                            nf[k] = vals.load(k, row + BLOCK);
-                            nbk[k] = vals.load(k, row + BLOCK - A.off[k]);
+                            nv[k] = vals.load(k, row + BLOCK);
+                            nvb[k] = vals.load(k, row + BLOCK - A.off[k]);
                         }
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);
+                T a0 = T(0), a1 = T(0);
+                const int jk = j < NK ? j : 0;
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    a0 += sf[k] * (win[A.lf[k] + l] - p[j]);
-                    a1 += sb[k] * (win[A.lb[k] + l] - p[j]);
+                    a0 += (j < NK ? vf[jk][k] : sf[k]) * (pf[k] - p[j]);
+                    a1 += (j < NK ? vb[jk][k] : sb[k]) * (pb[k] - p[j]);
                 }
-                if (j + 1 < RPT) {
+                if (AHEAD && j + 1 < RPT) {
 #pragma unroll
                     for (int k = 0; k < K; ++k) {
-                        sf[k] = nf[k];
-                        sb[k] = nbk[k];
+                        pf[k] = nf[k];
+                        pb[k] = nbk[k];
                     }
                 }
+                if (NK < RPT && j >= NK && j + 1 < RPT) {
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        sf[k] = nv[k];
+                        sb[k] = nvb[k];
+                    }
+                }
+                const T q = d[j] != T(0) ? a0 + a1 : T(0);
+                w[j] = d[j] * q;
+                rows.store(tag, row, w[j]);  // 0 past the last row
+                const double zd = static_cast<double>(z[j]), qd = static_cast<double>(q);
+                const double rd = static_cast<double>(g[j] * z[j]);
+                s[0] += static_cast<double>(p[j]) * qd;
+                s[1] += rd * zd;
+                s[2] += qd * zd;
+                s[3] += qd * static_cast<double>(w[j]);
+                s[4] += rd * rd;
+                __builtin_amdgcn_sched_barrier(0);
             }
-            const T q = d[j] != T(0) ? a0 + a1 : T(0);
-            w[j] = d[j] * q;
-            if (row < n) rows.store(tag, row, w[j]);
-            const double zd = static_cast<double>(z[j]), qd = static_cast<double>(q);
-            const double rd = static_cast<double>(g[j] * z[j]);
-            s[0] += static_cast<double>(p[j]) * qd;
-            s[1] += rd * zd;
-            s[2] += qd * zd;
-            s[3] += qd * static_cast<double>(w[j]);
-            s[4] += rd * rd;
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
-        T ww[U];
+            alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+            T ww[U];
+            const int32_t ft = fresh(tid);
 #pragma unroll
-        for (int u = 0; u < U; ++u) ww[u] = rows.load(tag, window_row(A, i0, fresh(li[u])));
-        const double pq = s[0], rz = s[1];
-        const T alpha = static_cast<T>(rz / pq);
-        const double al = static_cast<double>(alpha), inv_rz = 1.0 / rz;
-        const T beta = static_cast<T>(fmax(rz - al * (2.0 * s[2] - al * s[3]), 0.0) * inv_rz);
-        rr = s[4];
-        if (it == 0) {
-            if (!(bb >= 0.0)) bb = rr;
-            thresh = A.rtol * A.rtol * bb;
-        }
-        code = !alive                                      ? FK_ERR_HIP
-               : rr < thresh || (it == 0 && rr == 0.0)     ? FK_OK
-               : !isfinite(rr)                             ? FK_ERR_NONFINITE
-               : it >= A.max_iter                          ? FK_ERR_NOT_CONVERGED
-               : !(pq > 0.0) || !isfinite(pq)              ? FK_ERR_SINGULAR  // not positive definite on the space
-                                                           : -1;
-        code = __builtin_amdgcn_readfirstlane(code);
-        if (code >= 0) break;
-        ++it;
+            for (int u = 0; u < U; ++u) ww[u] = rows.load(tag, window_row(A, i0, window_lds(A, R, ft + u * BLOCK)));
+            const double pq = s[0], rz = s[1];
+            const T alpha = static_cast<T>(rz / pq);
+            const double al = static_cast<double>(alpha), inv_rz = 1.0 / rz;
+            const T beta = static_cast<T>(fmax(rz - al * (2.0 * s[2] - al * s[3]), 0.0) * inv_rz);
+            rr = s[4];
+            if constexpr (REFINE) {
+                act = !alive                                                   ? 3
+                      : moved && rr < A.target2                                ? 1
+                      : !isfinite(rr)                                          ? 2
+                      : it >= A.max_iter                                       ? 1
+                      : until_check == 0 && moved && rr < A.delta2 * rr_last   ? 1
+                      : !(pq > 0.0) || !isfinite(pq)                           ? 2
+                                                                               : 0;
+                act = __builtin_amdgcn_readfirstlane(act);
+                if (until_check == 0) until_check = A.G;
+                if (act) break;
+                --until_check;
+                moved = true;
+            } else {
+                if (it == 0) {
+                    if (!(bb >= 0.0)) bb = rr;
+                    thresh = A.rtol * A.rtol * bb;
+                }
+                code = !alive                                  ? FK_ERR_HIP
+                       : rr < thresh || (it == 0 && rr == 0.0) ? FK_OK
+                       : !isfinite(rr)                         ? FK_ERR_NONFINITE
+                       : it >= A.max_iter                      ? FK_ERR_NOT_CONVERGED
+                       : !(pq > 0.0) || !isfinite(pq)          ? FK_ERR_SINGULAR  // not positive definite on the space
+                                                               : -1;
+                code = __builtin_amdgcn_readfirstlane(code);
+                if (code >= 0) break;
+            }
+            ++it;
 #pragma unroll
-        for (int j = 0; j < RPT; ++j) {
-            x[j] += alpha * p[j];
-            z[j] -= alpha * w[j];
-            p[j] = z[j] + beta * p[j];
-            win[A.lown + j * BLOCK + tid] = p[j];
-        }
+            for (int j = 0; j < RPT; ++j) {
+                (XLDS ? xs[j * BLOCK + ft] : x[XLDS ? 0 : j]) += alpha * p[j];
+                z[j] -= alpha * w[j];
+                p[j] = z[j] + beta * p[j];
+                win[A.lown + j * BLOCK + ft] = p[j];
+            }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            zw[u] -= alpha * ww[u];
-            win[li[u]] = zw[u] + beta * win[li[u]];
+            for (int u = 0; u < U; ++u) {
+                const int32_t li = window_lds(A, R, ft + u * BLOCK);
+                zw[u] -= alpha * ww[u];
+                win[li] = zw[u] + beta * win[li];
+            }
+            __syncthreads();
         }
-        __syncthreads();
-    }
+        if constexpr (!REFINE) {
 #pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int32_t row = i0 + j * BLOCK + tid;
-        if (row < n) A.x[row] = x[j];
+            for (int j = 0; j < RPT; ++j) {
+                const int32_t row = i0 + j * BLOCK + tid;
+                if (row < n) A.x[row] = XLDS ? xs[j * BLOCK + tid] : x[XLDS ? 0 : j];
+            }
+        } else {
+            static_assert(!XLDS, "the replacement folds x from registers");
+            // ---- replacement: nothing but x and p leaves the registers
+            if (act == 3) {
+                code = FK_ERR_HIP;
+                break;
+            }
+            restart = act == 2;
+            const int32_t tc = fresh(tid);
+            const AgentRows<double> sol(A.u, n);
+            if (act == 1) {
+                const double inv_s = 1.0 / A.s;
+#pragma unroll
+                for (int j = 0; j < RPT; ++j) {
+                    const int32_t row = i0 + j * BLOCK + tc;
+                    if (row < n) {
+                        sol.store(0, row, A.u[row] + inv_s * static_cast<double>(x[XLDS ? 0 : j]));
+                        A.p[row] = p[j];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                ++tag;
+                alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+                // the other blocks' u through this CU's caches: one wave's
+                // acquire serves the block (a fence in every wave takes 16
+                // times as long)
+                if (tid < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                __syncthreads();
+            } else {
+                if (++restarts > kResRestarts || it >= A.max_iter) {
+                    code = it >= A.max_iter ? FK_ERR_NOT_CONVERGED : isfinite(rr) ? FK_ERR_SINGULAR : FK_ERR_NONFINITE;
+                    break;
+                }
+                ++it;
+            }
+            ++tag;
+            s[0] = 0.0;
+#pragma unroll 1
+            for (int j = 0; j < RPT; ++j) {
+                const int32_t row = i0 + j * BLOCK + tc;
+                if (row >= n) continue;
+                const T dj = A.dinv[row];
+                double v = dj != T(0) ? A.r64[row] : 0.0;
+                if (act == 1) {
+                    double y0 = 0.0, y1 = 0.0;
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (k < A.K) {
+                            const int32_t o = A.off[k], f = min(row + o, n - 1), bk = max(row - o, 0);
+                            const double *__restrict__ c = A.val64 + static_cast<int64_t>(k) * A.ld;
+                            const double vb64 = c[bk];
+                            y0 += c[row] * A.u[f];  // 0 where row + o is past the last row
+                            y1 += (row >= o ? vb64 : 0.0) * A.u[bk];
+                        }
+                    const double y = (y0 + y1) + A.diag64[row] * A.u[row];
+                    v = dj != T(0) ? (A.b ? A.b[row] - y : -y) : 0.0;
+                    A.r64[row] = v;
+                    s[0] += v * v;
+                }
+                rows.store(tag, row, dj * static_cast<T>(A.s * v));
+            }
+            alive = alive && all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+            if (!alive) {
+                code = FK_ERR_HIP;
+                break;
+            }
+            if (act == 1) {
+                rr64 = s[0];
+                ++nrep;
+                rr_last = rr64 * A.s * A.s;
+                restart = rr_last > 4.0 * rr;  // the recursion drifted below the true residual
+                if (restart && !(rr64 < A.thresh64)) ++restarts;
+                code = rr64 < A.thresh64                             ? FK_OK
+                       : !isfinite(rr64)                             ? FK_ERR_NONFINITE
+                       : it >= A.max_iter || restarts > kResRestarts ? FK_ERR_NOT_CONVERGED
+                                                                     : -1;
+                code = __builtin_amdgcn_readfirstlane(code);
+                restart = __builtin_amdgcn_readfirstlane(restart);
+            }
+        }
     }
     if (blockIdx.x == 0 && tid == 0) {
+        if constexpr (REFINE) {
+            A.ru->nrep = nrep;
+            A.ru->restarts = restarts;
+            A.ru->rr64 = rr64;
+            A.ru->status = code;
+        }
         A.state->iters = it;
         A.state->rr = rr;
         A.state->bb = bb;
@@ -305,31 +474,32 @@ static bool place_windows(const fk_mesh *m, int R, ResidentArgs<T> &A, int32_t *
     return true;
 }
 
-template <typename T, int BLOCK, int RPT, int NK>
+template <typename T, int BLOCK, int RPT, int NK, bool REFINE = false>
 static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     constexpr int R = BLOCK * RPT, U = 2 * RPT + 2;
     const int most = std::min(m->ctx->num_cus, kMaxResidentBlocks);
     int nb = static_cast<int>((m->nv + R - 1) / R);
+    if (nb > most) return false;
     // streamed values: one band of rows per XCD
     if (NK < RPT && nb > kNumXcd) nb = std::min((nb + kNumXcd - 1) / kNumXcd * kNumXcd, most);
     int32_t elements = 0;
     if (!place_windows<T>(m, R, A, &elements) || elements - R > U * BLOCK) return false;
-    const size_t lds = (static_cast<size_t>(elements) + 1) * sizeof(T);
+    const size_t lds = (static_cast<size_t>(elements) + 1 + (x_in_lds<T>(RPT) ? R : 0)) * sizeof(T);
     if (lds > static_cast<size_t>(kResLdsMax)) return false;
     A.nb = nb;
     // rows past the last, as far as the last block's windows reach, read zero
     const int64_t reach = static_cast<int64_t>(nb) * R + m->st_off[m->st_K - 1] + R;
     const int64_t stride = (reach + 63) / 64 * 64;
     hipStream_t st = m->ctx->stream;
-    m->res_slots.ensure(reduce_words(5));
+    m->res_slots.ensure(kReduceWords);
     m->res_w.ensure(static_cast<size_t>(2 * stride));
     A.stride = static_cast<int32_t>(stride);
     A.slots = m->res_slots.get();
     A.w = reinterpret_cast<T *>(m->res_w.get());
-    auto kern = k_resident_pcg<T, BLOCK, RPT, NK, U>;
+    auto kern = k_resident_pcg<T, BLOCK, RPT, NK, U, REFINE>;
     FK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                static_cast<int>(lds)));
-    k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, reduce_words(5), A.w, A.n, A.stride);
+    k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, kReduceWords, A.w, A.n, A.stride);
     FK_HIP(hipGetLastError());
     void *args[] = {&A};
     const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kern), dim3(nb), dim3(BLOCK),
@@ -347,29 +517,53 @@ static std::mutex &resident_mutex(int device) {
     return all[device & 63];
 }
 
-// Rows per block R by the number of rows: the smallest of the list with which
-// at most one block per CU covers them. Few rows per thread leave room for all
-// their matrix values in registers (NK = RPT) and shorten every step between
-// two exchanges; beyond 5 per thread the values are streamed. Measured per
-// iteration (us; three-kernel iteration in brackets), Kuhn meshes of n cells
-// per side:
-//   n = 20  512 x 1   4.1 (14.7)     n = 40  512 x 1   4.3 (15.9)
-//   n = 60 1024 x 1   5.2 (21.0)     n = 70  512 x 4  10.5 (23.7)
-//   n = 79  512 x 4  11.9 (26.9)     n = 85  512 x 5  14.6 (29.4)
-//   n = 92  512 x 8  20.6 (32.6)     n = 100 512 x 8  25.1 (36.8)
-// More rows than 256 blocks of 4096 keep the three-kernel iteration: the
-// windows of more rows per block exceed the LDS.
+static int64_t rows_per_block(const fk_mesh *m) {
+    const int most = std::min(m->ctx->num_cus, kMaxResidentBlocks);
+    return (m->nv + most - 1) / most;
+}
+
+// Rows per block by the number of rows: the smallest shape of the list with
+// which at most one block per CU covers them. Few rows per thread leave room
+// for all their matrix values in registers (NK = RPT) and shorten every step
+// between two exchanges. Measured per iteration (us; three-kernel iteration in
+// brackets), Kuhn meshes of n cells per side:
+//   n = 20  512 x 1   3.9 (14.7)     n = 40  512 x 1   4.2 (15.9)
+//   n = 63  512 x 2   4.8 (21.5)     n = 70  512 x 3   6.4 (23.7)
+//   n = 79  512 x 4   7.6 (26.9)     n = 85  512 x 5  11.3 (29.4)
+//   n = 90  512 x 6  14.5 (31.5)     n = 95  512 x 7  17.8 (34)
+//   n = 100 512 x 8  21.8 (36.8)
+// One shape up costs: n = 63 on 512 x 3 5.8, n = 79 on 512 x 5 10.9, n = 85 on
+// 512 x 6 13.6. More rows than 256 blocks of 4096 keep the three-kernel
+// iteration: the windows of more rows per block exceed the LDS.
 static bool launch_by_rows(fk_mesh *m, ResidentArgs<double> &A) {
-    const int64_t per = (m->nv + std::min(m->ctx->num_cus, kMaxResidentBlocks) - 1) /
-                        std::min(m->ctx->num_cus, kMaxResidentBlocks);
+    const int64_t per = rows_per_block(m);
     if (per <= 512) return launch_resident<double, 512, 1, 1>(m, A);
-    if (per <= 1024) return launch_resident<double, 1024, 1, 1>(m, A);
+    if (per <= 1024) return launch_resident<double, 512, 2, 2>(m, A);
     if (per <= 1536) return launch_resident<double, 512, 3, 3>(m, A);
-    if (per <= 2048) return launch_resident<double, 512, 4, 3>(m, A);
-    if (per <= 2560) return launch_resident<double, 512, 5, 3>(m, A);
+    if (per <= 2048) return launch_resident<double, 512, 4, 4>(m, A);
+    if (per <= 2560) return launch_resident<double, 512, 5, 2>(m, A);
     if (per <= 3072) return launch_resident<double, 512, 6, 1>(m, A);
     if (per <= 3584) return launch_resident<double, 512, 7, 0>(m, A);
     if (per <= 4096) return launch_resident<double, 512, 8, 0>(m, A);
+    return false;
+}
+
+// The same for the FP32 recursion with residual replacement, half the
+// registers and LDS per row. Measured as above, replacements included:
+//   n = 20  512 x 1   4.2 (14.5)     n = 48  512 x 1   5.1 (15.7)
+//   n = 63  512 x 2   5.2 (19.0)     n = 75  512 x 4   6.9 (20.7)
+//   n = 90 1024 x 3   9.7 (22.8)     n = 100 512 x 8  13.7 (25.2)
+//   n = 115 512 x 12 20   (31)       n = 126 512 x 16 28.1 (35.6)
+static bool launch_by_rows(fk_mesh *m, ResidentArgs<float> &A) {
+    const int64_t per = rows_per_block(m);
+    if (per <= 512) return launch_resident<float, 512, 1, 1, true>(m, A);
+    if (per <= 1024) return launch_resident<float, 512, 2, 2, true>(m, A);
+    if (per <= 1536) return launch_resident<float, 512, 3, 3, true>(m, A);
+    if (per <= 2048) return launch_resident<float, 512, 4, 4, true>(m, A);
+    if (per <= 3072) return launch_resident<float, 1024, 3, 3, true>(m, A);
+    if (per <= 4096) return launch_resident<float, 512, 8, 8, true>(m, A);
+    if (per <= 6144) return launch_resident<float, 512, 12, 4, true>(m, A);
+    if (per <= 8192) return launch_resident<float, 512, 16, 0, true>(m, A);
     return false;
 }
 
@@ -398,6 +592,53 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
     FK_HIP(hipStreamSynchronize(st));
     if (hs->status == FK_ERR_HIP) return false;  // a wait ran out (another process's launch); r0 is unchanged
     *out = *hs;
+    return true;
+}
+
+// The FP32-refined solve of solve.hip's solve_f32_replace from the FP64
+// residual in r64 (its norm^2 rr): false when this mesh or moment does not
+// allow a resident launch; u and r64 may then have changed.
+bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
+                      int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status) {
+    if (m->kind != FK_SPMV_STENCIL || m->st_K > kResK || m->ctx->timing.enabled) return false;
+    PcgWork<float> &w = m->w32;
+    if (!m->ru) {
+        m->ru.alloc(1);
+        m->hru.alloc(2);
+    }
+    ResidentArgs<float> A{};
+    A.val = m->st_val32.get();
+    A.dinv = w.dinv.get();
+    A.state = w.state.get();
+    A.ld = static_cast<int32_t>(m->st_ld);
+    A.n = static_cast<int32_t>(m->nv);
+    A.K = m->st_K;
+    A.max_iter = max_iter;
+    A.u = u;
+    A.b = b;
+    A.r64 = m->r64.get();
+    A.val64 = m->st_val64.get();
+    A.diag64 = m->sell_diag64.get();
+    A.ru = m->ru.get();
+    A.p = w.p.get();
+    A.s = 1.0 / std::sqrt(rr);
+    A.target2 = thresh * A.s * A.s;
+    A.thresh64 = thresh;
+    A.delta2 = delta * delta;
+    A.G = chunk;
+    const std::lock_guard<std::mutex> alone(resident_mutex(m->ctx->device));
+    if (!launch_by_rows(m, A)) return false;
+    hipStream_t st = m->ctx->stream;
+    CgState *hs = m->hstate.ptr;
+    RuState *hr = m->hru.ptr;
+    FK_HIP(hipMemcpyAsync(hs, w.state.get(), sizeof(CgState), hipMemcpyDeviceToHost, st));
+    FK_HIP(hipMemcpyAsync(hr, m->ru.get(), sizeof(RuState), hipMemcpyDeviceToHost, st));
+    FK_HIP(hipStreamSynchronize(st));
+    if (hr->status == FK_ERR_HIP) return false;  // a wait ran out (another process's launch)
+    *iters = hs->iters;
+    *nrep = hr->nrep;
+    *rr_out = hr->rr64;
+    *status = hr->status;
     return true;
 }
 

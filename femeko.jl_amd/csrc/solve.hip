@@ -1888,9 +1888,15 @@ static int solve_f32_replace(fk_mesh *m, double *u, const double *b, double rtol
     *nrep = 0;
     *rr_out = rr;
     if (rr < thresh) return FK_OK;
+    const int G = nv > 200000 ? 32 : 16;
+    sync_solver_values<float>(m);
+    if (std::isfinite(rr)) {
+        int status = FK_OK;
+        if (resident_refined(m, u, b, rr, thresh, delta, max_iter, G, iters, nrep, rr_out, &status)) return status;
+        rr = neg_residual(m, u, m->r64.get(), b);
+    }
     const double s = 1.0 / std::sqrt(rr);
     const double target2 = thresh * s * s;
-    sync_solver_values<float>(m);
     k_scale_to_f32<<<grid_for(nv, 256), 256, 0, st>>>(m->r64.get(), w.r.get(), s, nv);
     k_cg_init<float><<<nb, kBlock, 0, st>>>(w.x.get(), w.r.get(), w.p.get(), w.dinv.get(), w.part_rz.get(),
                                             w.part_bb.get(), nv, m->chunk, nb);
@@ -1911,7 +1917,6 @@ static int solve_f32_replace(fk_mesh *m, double *u, const double *b, double rtol
     init.delta2 = delta * delta;
     FK_HIP(hipMemcpyAsync(m->ru.get(), &init, sizeof(RuState), hipMemcpyHostToDevice, st));
     m->part_misc.ensure(nb);
-    const int G = nv > 200000 ? 32 : 16;
     const char *tr = std::getenv("FEMEKO_HIP_TRACE");
     const bool trace = tr && tr[0] == '1';
     const bool timed = m->ctx->timing.enabled;
