@@ -290,6 +290,11 @@ struct fk_mesh {
     // register-resident PCG (resident.hip): all-reduce slots, exchanged row values
     fk::DevBuf<unsigned long long> res_slots;
     fk::DevBuf<double> res_w;
+    // and its lists on the SELL copy: rows per block (0: none), longest row and
+    // halo, LDS index per entry, halo rows per block
+    int32_t res_R = 0, res_width = 0, res_halo_max = 0;
+    fk::DevBuf<uint16_t> res_sidx;
+    fk::DevBuf<int32_t> res_halo_ptr, res_halo;
 
     fk::PcgWork<double> w64;
     fk::PcgWork<float> w32;
@@ -337,6 +342,9 @@ inline void values_changed(fk_mesh *m) {
 }
 // FP64 PCG in one cooperative launch (resident.hip); false: not for this mesh
 bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, CgState *out);
+void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::vector<int32_t> &ci,
+                         const std::vector<int32_t> &width, const std::vector<std::vector<int32_t>> &shared,
+                         const std::vector<int64_t> &vptr);
 // the same for the FP32 recursion with FP64 residual replacement
 bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
                       int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status);

@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -55,6 +56,13 @@ struct ResidentArgs {
     int32_t lown;                 // LDS index of local row 0
     int32_t wbeg[kResWindows + 1];// LDS index of each window's first element; the number of elements
     int32_t wrow[kResWindows];    // row - i0 of an element - its LDS index, by window
+    // SELL copy (any pattern): LDS index of every entry, laid out like the
+    // values, and each block's list of rows outside its own (its halo)
+    const int64_t *sptr;
+    const int32_t *swidth;
+    const uint16_t *sidx;
+    const int32_t *halo_ptr, *halo;
+    int32_t nslices, spare;       // LDS index of the spare element
     double bb_ref, rtol;
     int64_t max_iter;
     // residual replacement (FP32 recursion, FP64 solution u)
@@ -101,6 +109,10 @@ constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursio
 // others are streamed from L2 / MALL, a row ahead of their use); U window
 // elements per thread at most.
 //
+// NE > 0: the SELL copy instead of the stencil, rows of at most NE entries.
+// The own rows lie first in LDS, the rows of the block's halo list after them,
+// and every entry keeps its value and the LDS index of its column.
+//
 // REFINE (T = float): the reliable updates of solve.hip inside the launch. At
 // the end of every G iterations in which ||r||^2 has fallen by delta2 since
 // the last replacement, and when the recursion has reached its target, x / s
@@ -108,21 +120,26 @@ constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursio
 // rows replaces the recursion's (times s), and p is kept; a recursion that has
 // drifted below the true residual, or broken down, restarts from p = z. The
 // solve ends on the FP64 residual.
-template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE>
+template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE, int NE>
 __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A) {
     extern __shared__ char lds_raw[];
     T *win = reinterpret_cast<T *>(lds_raw);
     __shared__ double sh[kReduceShared];
     constexpr int K = kResK, R = BLOCK * RPT;
+    constexpr bool GEN = NE > 0;
+    constexpr int E = GEN ? NE : 2 * K;  // entries per row: K forward, then K backward ones
+    static_assert(!GEN || NK == RPT, "SELL values are not streamed");
     // x of the FP64 shapes with many rows per thread waits in LDS, past the windows
     constexpr bool XLDS = x_in_lds<T>(RPT);
-    T *xs = win + A.wbeg[kResWindows] + 1;
-    constexpr bool AHEAD = RPT > 1 && (sizeof(T) == 4 || RPT <= 3);
+    T *xs = win + (GEN ? A.spare : A.wbeg[kResWindows]) + 1;
+    constexpr bool AHEAD = RPT > 1 && (sizeof(T) == 4 || (!GEN && RPT <= 3));
     const int32_t i0 = logical_block(A.nb) * R;
     const int32_t tid = threadIdx.x;
     const AgentRows<T> rows(A.w, A.stride);
     const ValueColumns<T> vals(A.val, A.K, A.ld);
-    const int32_t n = A.n;
+    const int32_t n = A.n, lown = GEN ? 0 : A.lown;
+    const int32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int32_t h0 = GEN ? A.halo_ptr[i0 / R] : 0, nh = GEN ? A.halo_ptr[i0 / R + 1] - h0 : 0;
     uint32_t tag = 1;
     if (tid == 0) sh[kReduceShared - 1] = 0.0;
 
@@ -150,7 +167,31 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
         const int32_t tl = fresh(tid);
         T d[RPT], g[RPT], x[XLDS ? 1 : RPT], z[RPT], p[RPT], w[RPT];
         T zw[U];
-        T vf[NK > 0 ? NK : 1][K], vb[NK > 0 ? NK : 1][K];
+        T v[NK > 0 ? NK : 1][E];
+        [[maybe_unused]] uint32_t pk[GEN ? RPT : 1][GEN ? NE / 2 : 1];  // LDS indices of two entries
+        [[maybe_unused]] int32_t hrow[GEN ? U : 1];                     // rows of this thread's halo elements
+        // LDS index and row of the u-th window element (spare: none)
+        const auto element = [&](int u, int32_t t, int32_t &row) {
+            if constexpr (GEN) {
+                row = hrow[u];
+                return row >= 0 ? R + t + u * BLOCK : A.spare;
+            } else {
+                const int32_t li = window_lds(A, R, t + u * BLOCK);
+                row = window_row(A, i0, li);
+                return li;
+            }
+        };
+        // the value pairs of a row of the stencil
+        const auto load_row = [&](int32_t row, T(&o)[E]) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                o[k] = o[K + k] = T(0);
+                if (k < A.K) {
+                    o[k] = vals.load(k, row);
+                    o[K + k] = vals.load(k, row - A.off[k]);
+                }
+            }
+        };
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
             const int32_t row = i0 + j * BLOCK + tl, at = min(row, n - 1);
@@ -162,24 +203,45 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                 xs[j * BLOCK + tl] = T(0);
             else
                 (XLDS ? xs[j * BLOCK + tl] : x[XLDS ? 0 : j]) = T(0);
-            if (restart) win[A.lown + j * BLOCK + tl] = p[j];
+            if (restart) win[lown + j * BLOCK + tl] = p[j];
         }
 #pragma unroll
         for (int j = 0; j < RPT; ++j) g[j] = d[j] != T(0) ? T(1) / d[j] : T(0);
+        if constexpr (GEN) {
 #pragma unroll
-        for (int j = 0; j < NK; ++j)
+            for (int j = 0; j < RPT; ++j) {
+                const int32_t sl = i0 / 64 + j * (BLOCK / 64) + wave, own = j * BLOCK + tl;
+                const bool in = sl < A.nslices;
+                const int64_t base = in ? A.sptr[sl] : 0;
+                const int32_t W = in ? abs(A.swidth[sl]) : 0, ng = W >> 2, lane = tl & 63;
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                vf[j][k] = vb[j][k] = T(0);
-                if (k < A.K) {
-                    vf[j][k] = vals.load(k, i0 + j * BLOCK + tl);
-                    vb[j][k] = vals.load(k, i0 + j * BLOCK + tl - A.off[k]);
+                for (int k = 0; k < NE; ++k) {
+                    T a = T(0);
+                    uint32_t ix = static_cast<uint32_t>(own);
+                    if (k < W) {
+                        const int64_t at = base + (k < 4 * ng ? 4 * (64 * (k >> 2) + lane) + (k & 3)
+                                                              : 256 * ng + 64 * (k - 4 * ng) + lane);
+                        a = A.val[at];
+                        ix = A.sidx[at];
+                    }
+                    v[j][k] = a;
+                    pk[j][k / 2] = (k & 1) ? pk[j][k / 2] | ix << 16 : ix;
                 }
             }
 #pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int32_t e = tl + u * BLOCK;
+                hrow[u] = e < nh ? A.halo[h0 + e] : -1;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NK; ++j) load_row(i0 + j * BLOCK + tl, v[j]);
+        }
+#pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int32_t li = window_lds(A, R, tl + u * BLOCK);
-            zw[u] = rows.load(tag, window_row(A, i0, li));
+            int32_t row;
+            const int32_t li = element(u, tl, row);
+            zw[u] = rows.load(tag, row);
             if (restart) win[li] = zw[u];
         }
         __syncthreads();
@@ -190,67 +252,48 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
             // q = A p in difference form; w = D^-1 q
 #pragma unroll
             for (int k = 0; k < 5; ++k) s[k] = 0.0;
-            T sf[K], sb[K];
-            [[maybe_unused]] const int32_t t0 = fresh(tid);
-            if constexpr (NK < RPT) {
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    sf[k] = sb[k] = T(0);
-                    if (k < A.K) {
-                        sf[k] = vals.load(k, i0 + NK * BLOCK + t0);
-                        sb[k] = vals.load(k, i0 + NK * BLOCK + t0 - A.off[k]);
-                    }
-                }
-            }
+            [[maybe_unused]] T sv[E];  // values of the streamed row at hand
+            if constexpr (NK < RPT) load_row(i0 + NK * BLOCK + fresh(tid), sv);
             // the neighbours of a row are loaded together, and where registers
             // allow a row ahead: one LDS latency per row, not one per neighbour
-            T pf[K], pb[K];
-            const auto neighbours = [&](int j, T(&f)[K], T(&b)[K]) {
-                const int32_t l = j * BLOCK + fresh(tid);
+            T nb[E];
+            const auto neighbours = [&](int j, T(&o)[E]) {
+                if constexpr (GEN) {
 #pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    f[k] = win[A.lf[k] + l];
-                    b[k] = win[A.lb[k] + l];
+                    for (int k = 0; k < NE; ++k)
+                        o[k] = win[(k & 1) ? pk[j][k / 2] >> 16 : pk[j][k / 2] & 0xffffu];
+                } else {
+                    const int32_t l = j * BLOCK + fresh(tid);
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        o[k] = win[A.lf[k] + l];
+                        o[K + k] = win[A.lb[k] + l];
+                    }
                 }
             };
-            if constexpr (AHEAD) neighbours(0, pf, pb);
+            if constexpr (AHEAD) neighbours(0, nb);
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
                 const int32_t row = i0 + j * BLOCK + fresh(tid);
-                T nf[K], nbk[K], nv[K], nvb[K];
-                if (AHEAD && j + 1 < RPT) neighbours(j + 1, nf, nbk);
-                if (!AHEAD) neighbours(j, pf, pb);
-                if (NK < RPT && j >= NK && j + 1 < RPT) {
-#pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        nv[k] = nvb[k] = T(0);
-                        if (k < A.K) {
-                            nv[k] = vals.load(k, row + BLOCK);
-                            nvb[k] = vals.load(k, row + BLOCK - A.off[k]);
-                        }
-                    }
-                }
+                T next[E], nv[E];
+                if (AHEAD && j + 1 < RPT) neighbours(j + 1, next);
+                if (!AHEAD) neighbours(j, nb);
+                if (NK < RPT && j >= NK && j + 1 < RPT) load_row(row + BLOCK, nv);
                 __builtin_amdgcn_sched_barrier(0);
                 T a0 = T(0), a1 = T(0);
                 const int jk = j < NK ? j : 0;
 #pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    a0 += (j < NK ? vf[jk][k] : sf[k]) * (pf[k] - p[j]);
-                    a1 += (j < NK ? vb[jk][k] : sb[k]) * (pb[k] - p[j]);
+                for (int k = 0; k < E / 2; ++k) {
+                    a0 += (j < NK ? v[jk][k] : sv[k]) * (nb[k] - p[j]);
+                    a1 += (j < NK ? v[jk][E / 2 + k] : sv[E / 2 + k]) * (nb[E / 2 + k] - p[j]);
                 }
                 if (AHEAD && j + 1 < RPT) {
 #pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        pf[k] = nf[k];
-                        pb[k] = nbk[k];
-                    }
+                    for (int k = 0; k < E; ++k) nb[k] = next[k];
                 }
                 if (NK < RPT && j >= NK && j + 1 < RPT) {
 #pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        sf[k] = nv[k];
-                        sb[k] = nvb[k];
-                    }
+                    for (int k = 0; k < E; ++k) sv[k] = nv[k];
                 }
                 const T q = d[j] != T(0) ? a0 + a1 : T(0);
                 w[j] = d[j] * q;
@@ -268,7 +311,11 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
             T ww[U];
             const int32_t ft = fresh(tid);
 #pragma unroll
-            for (int u = 0; u < U; ++u) ww[u] = rows.load(tag, window_row(A, i0, window_lds(A, R, ft + u * BLOCK)));
+            for (int u = 0; u < U; ++u) {
+                int32_t row;
+                (void)element(u, ft, row);
+                ww[u] = rows.load(tag, row);
+            }
             const double pq = s[0], rz = s[1];
             const T alpha = static_cast<T>(rz / pq);
             const double al = static_cast<double>(alpha), inv_rz = 1.0 / rz;
@@ -307,11 +354,12 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                 (XLDS ? xs[j * BLOCK + ft] : x[XLDS ? 0 : j]) += alpha * p[j];
                 z[j] -= alpha * w[j];
                 p[j] = z[j] + beta * p[j];
-                win[A.lown + j * BLOCK + ft] = p[j];
+                win[lown + j * BLOCK + ft] = p[j];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int32_t li = window_lds(A, R, ft + u * BLOCK);
+                int32_t row;
+                const int32_t li = element(u, ft, row);
                 zw[u] -= alpha * ww[u];
                 win[li] = zw[u] + beta * win[li];
             }
@@ -368,15 +416,28 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                 double v = dj != T(0) ? A.r64[row] : 0.0;
                 if (act == 1) {
                     double y0 = 0.0, y1 = 0.0;
-#pragma unroll
-                    for (int k = 0; k < K; ++k)
-                        if (k < A.K) {
-                            const int32_t o = A.off[k], f = min(row + o, n - 1), bk = max(row - o, 0);
-                            const double *__restrict__ c = A.val64 + static_cast<int64_t>(k) * A.ld;
-                            const double vb64 = c[bk];
-                            y0 += c[row] * A.u[f];  // 0 where row + o is past the last row
-                            y1 += (row >= o ? vb64 : 0.0) * A.u[bk];
+                    if constexpr (GEN) {
+                        const int32_t sl = i0 / 64 + j * (BLOCK / 64) + wave, lane = tc & 63;
+                        const int64_t base = A.sptr[sl];
+                        const int32_t W = abs(A.swidth[sl]), ng = W >> 2;
+#pragma unroll 4
+                        for (int k = 0; k < W; ++k) {
+                            const int64_t at = base + (k < 4 * ng ? 4 * (64 * (k >> 2) + lane) + (k & 3)
+                                                                  : 256 * ng + 64 * (k - 4 * ng) + lane);
+                            const int32_t ix = A.sidx[at];
+                            y0 += A.val64[at] * A.u[ix < R ? i0 + ix : A.halo[h0 + ix - R]];
                         }
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < K; ++k)
+                            if (k < A.K) {
+                                const int32_t o = A.off[k], f = min(row + o, n - 1), bk = max(row - o, 0);
+                                const double *__restrict__ c = A.val64 + static_cast<int64_t>(k) * A.ld;
+                                const double vb64 = c[bk];
+                                y0 += c[row] * A.u[f];  // 0 where row + o is past the last row
+                                y1 += (row >= o ? vb64 : 0.0) * A.u[bk];
+                            }
+                    }
                     const double y = (y0 + y1) + A.diag64[row] * A.u[row];
                     v = dj != T(0) ? (A.b ? A.b[row] - y : -y) : 0.0;
                     A.r64[row] = v;
@@ -474,21 +535,33 @@ static bool place_windows(const fk_mesh *m, int R, ResidentArgs<T> &A, int32_t *
     return true;
 }
 
-template <typename T, int BLOCK, int RPT, int NK, bool REFINE = false>
+template <typename T, int BLOCK, int RPT, int NK, bool REFINE = false, int NE = 0>
 static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
-    constexpr int R = BLOCK * RPT, U = 2 * RPT + 2;
+    constexpr int R = BLOCK * RPT, U = NE > 0 ? (RPT <= 2 ? 4 * RPT : 3 * RPT) : 2 * RPT + 2;
     const int most = std::min(m->ctx->num_cus, kMaxResidentBlocks);
     int nb = static_cast<int>((m->nv + R - 1) / R);
     if (nb > most) return false;
     // streamed values: one band of rows per XCD
     if (NK < RPT && nb > kNumXcd) nb = std::min((nb + kNumXcd - 1) / kNumXcd * kNumXcd, most);
     int32_t elements = 0;
-    if (!place_windows<T>(m, R, A, &elements) || elements - R > U * BLOCK) return false;
+    if constexpr (NE > 0) {
+        if (m->res_R != R || m->res_halo_max > U * BLOCK) return false;
+        elements = R + m->res_halo_max;
+        A.spare = elements;
+        A.sptr = m->sell_ptr.get();
+        A.swidth = m->sell_width.get();
+        A.sidx = m->res_sidx.get();
+        A.halo_ptr = m->res_halo_ptr.get();
+        A.halo = m->res_halo.get();
+        A.nslices = static_cast<int32_t>(m->nslices);
+    } else {
+        if (!place_windows<T>(m, R, A, &elements) || elements - R > U * BLOCK) return false;
+    }
     const size_t lds = (static_cast<size_t>(elements) + 1 + (x_in_lds<T>(RPT) ? R : 0)) * sizeof(T);
     if (lds > static_cast<size_t>(kResLdsMax)) return false;
     A.nb = nb;
     // rows past the last, as far as the last block's windows reach, read zero
-    const int64_t reach = static_cast<int64_t>(nb) * R + m->st_off[m->st_K - 1] + R;
+    const int64_t reach = static_cast<int64_t>(nb) * R + (NE > 0 ? 0 : m->st_off[m->st_K - 1] + R);
     const int64_t stride = (reach + 63) / 64 * 64;
     hipStream_t st = m->ctx->stream;
     m->res_slots.ensure(kReduceWords);
@@ -496,7 +569,7 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     A.stride = static_cast<int32_t>(stride);
     A.slots = m->res_slots.get();
     A.w = reinterpret_cast<T *>(m->res_w.get());
-    auto kern = k_resident_pcg<T, BLOCK, RPT, NK, U, REFINE>;
+    auto kern = k_resident_pcg<T, BLOCK, RPT, NK, U, REFINE, NE>;
     FK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                static_cast<int>(lds)));
     k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, kReduceWords, A.w, A.n, A.stride);
@@ -567,11 +640,171 @@ static bool launch_by_rows(fk_mesh *m, ResidentArgs<float> &A) {
     return false;
 }
 
+// Rows per block of the SELL shapes (0: none): the same for both precisions.
+static int sell_rows_per_block(const fk_mesh *m, int width) {
+    const int64_t per = rows_per_block(m);
+    const int most = width <= 20 ? 2048 : width <= 32 ? 1024 : 0;
+    const int R = static_cast<int>((per + 511) / 512 * 512);
+    return R <= most ? R : 0;
+}
+
+// By the longest row (up to 16 entries: a numbering of a structured mesh; 20:
+// the same with slices padded to a common offset set; 32: Delaunay meshes) and
+// the rows per block. The values, LDS indices and halo of more rows do not fit
+// the registers. Measured per iteration (us; three-kernel iteration in
+// brackets), randomly numbered Kuhn meshes:
+//   FP64  n = 20 3.4 (14.0)  n = 41 3.7 (15.9)  n = 55 4.7 (24.4)  n = 70 7.7 (29.6)
+//   FP32  n = 20 4.3 (15.3)  n = 41 5.0 (17.4)  n = 55 6.6 (21.2)  n = 70 6.7 (24.8)
+static bool launch_sell(fk_mesh *m, ResidentArgs<double> &A) {
+    const int w = m->res_width;
+    switch (m->res_R) {
+        case 512:
+            return w <= 16   ? launch_resident<double, 512, 1, 1, false, 16>(m, A)
+                   : w <= 20 ? launch_resident<double, 512, 1, 1, false, 20>(m, A)
+                             : launch_resident<double, 512, 1, 1, false, 32>(m, A);
+        case 1024:
+            return w <= 16   ? launch_resident<double, 512, 2, 2, false, 16>(m, A)
+                   : w <= 20 ? launch_resident<double, 512, 2, 2, false, 20>(m, A)
+                             : false;
+        case 1536: return w <= 16 && launch_resident<double, 512, 3, 3, false, 16>(m, A);
+        default: return false;
+    }
+}
+
+static bool launch_sell(fk_mesh *m, ResidentArgs<float> &A) {
+    const int w = m->res_width;
+    switch (m->res_R) {
+        case 512:
+            return w <= 16   ? launch_resident<float, 512, 1, 1, true, 16>(m, A)
+                   : w <= 20 ? launch_resident<float, 512, 1, 1, true, 20>(m, A)
+                             : launch_resident<float, 512, 1, 1, true, 32>(m, A);
+        case 1024:
+            return w <= 16   ? launch_resident<float, 512, 2, 2, true, 16>(m, A)
+                   : w <= 20 ? launch_resident<float, 512, 2, 2, true, 20>(m, A)
+                             : launch_resident<float, 512, 2, 2, true, 32>(m, A);
+        case 1536:
+            return w <= 16 ? launch_resident<float, 512, 3, 3, true, 16>(m, A)
+                           : launch_resident<float, 512, 3, 3, true, 20>(m, A);
+        case 2048:
+            return w <= 16 ? launch_resident<float, 512, 4, 4, true, 16>(m, A)
+                           : launch_resident<float, 512, 4, 4, true, 20>(m, A);
+        default: return false;
+    }
+}
+
+// The LDS index of every SELL entry and the halo list of every block, from the
+// host's copy of the pattern while build_sell holds it. A block's halo is the
+// sorted set of the columns its rows have outside the block; on renumbered
+// meshes it is 2.2 to 2.5 times the block's rows. No lists are made (res_R = 0)
+// where the mesh is too large or its rows too long for the resident launch.
+void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::vector<int32_t> &ci,
+                         const std::vector<int32_t> &width, const std::vector<std::vector<int32_t>> &shared,
+                         const std::vector<int64_t> &vptr) {
+    m->res_R = 0;
+    const int64_t nv = m->nv, ns = static_cast<int64_t>(width.size());
+    int32_t most = 0;
+    for (int32_t w : width) most = std::max(most, w < 0 ? -w : w);
+    const int R = sell_rows_per_block(m, most);
+    if (!R || most == 0) return;
+    const int nb = static_cast<int>((nv + R - 1) / R);
+    std::vector<std::vector<int32_t>> halo(static_cast<size_t>(nb));
+    std::vector<uint16_t> idx(static_cast<size_t>(vptr[ns]));
+    const int nth = static_cast<int>(std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency())));
+    std::vector<std::thread> th;
+    bool fits = true;
+    std::mutex mu;
+    for (int q = 0; q < nth; ++q)
+        th.emplace_back([&, q] {
+            std::vector<int32_t> place(static_cast<size_t>(nv), -1);  // halo position of a row of the block at hand
+            for (int b = nb * q / nth; b < nb * (q + 1) / nth; ++b) {
+                const int64_t r0 = static_cast<int64_t>(b) * R, r1 = std::min(nv, r0 + R);
+                std::vector<int32_t> &h = halo[b];
+                for (int64_t k = rp[r0]; k < rp[r1]; ++k) {
+                    const int32_t c = ci[k];
+                    if ((c < r0 || c >= r1) && place[c] < 0) {
+                        place[c] = 0;
+                        h.push_back(c);
+                    }
+                }
+                std::sort(h.begin(), h.end());
+                if (h.size() + R > 0xfffe) {
+                    const std::lock_guard<std::mutex> lock(mu);
+                    fits = false;
+                    return;
+                }
+                for (size_t e = 0; e < h.size(); ++e) place[h[e]] = static_cast<int32_t>(e);
+                auto at = [&](int64_t c) {
+                    return static_cast<uint16_t>(c >= r0 && c < r1 ? c - r0 : R + place[c]);
+                };
+                for (int64_t s = r0 / 64; s < std::min(ns, (r0 + R) / 64); ++s) {
+                    const int32_t W = width[s] < 0 ? -width[s] : width[s], ng = W >> 2;
+                    for (int lane = 0; lane < 64; ++lane) {
+                        const int64_t r = s * 64 + lane;
+                        const uint16_t own = static_cast<uint16_t>(r - r0);
+                        const int32_t *lo = r < nv ? ci.data() + rp[r] : nullptr;
+                        const int32_t *hi = r < nv ? ci.data() + rp[r + 1] : nullptr;
+                        int32_t k = 0;
+                        auto put = [&](uint16_t v) {
+                            const int64_t o = k < 4 * ng ? 4 * (64 * static_cast<int64_t>(k >> 2) + lane) + (k & 3)
+                                                         : 256 * static_cast<int64_t>(ng) + 64 * (k - 4 * ng) + lane;
+                            idx[vptr[s] + o] = v;
+                            ++k;
+                        };
+                        if (width[s] < 0) {
+                            for (int32_t off : shared[s]) {
+                                const int64_t c = r + off;
+                                const int32_t *f = r < nv && c >= 0 && c < nv
+                                                       ? std::lower_bound(lo, hi, static_cast<int32_t>(c))
+                                                       : hi;
+                                put(f != hi && *f == c ? at(c) : own);
+                            }
+                        } else {
+                            for (const int32_t *c = lo; c != hi; ++c)
+                                if (*c != r) put(at(*c));
+                            while (k < W) put(own);
+                        }
+                    }
+                }
+                for (int32_t c : h) place[c] = -1;
+            }
+        });
+    for (auto &t : th) t.join();
+    if (!fits) return;
+    std::vector<int32_t> ptr(static_cast<size_t>(nb) + 1, 0), list;
+    int32_t hmax = 0;
+    for (int b = 0; b < nb; ++b) {
+        ptr[b + 1] = ptr[b] + static_cast<int32_t>(halo[b].size());
+        hmax = std::max(hmax, static_cast<int32_t>(halo[b].size()));
+        list.insert(list.end(), halo[b].begin(), halo[b].end());
+    }
+    hipStream_t st = m->ctx->stream;
+    m->res_sidx.alloc(idx.size());
+    m->res_halo_ptr.alloc(ptr.size());
+    m->res_halo.alloc(std::max<size_t>(list.size(), 1));
+    FK_HIP(hipMemcpyAsync(m->res_sidx.get(), idx.data(), idx.size() * sizeof(uint16_t), hipMemcpyHostToDevice, st));
+    FK_HIP(hipMemcpyAsync(m->res_halo_ptr.get(), ptr.data(), ptr.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    if (!list.empty())
+        FK_HIP(hipMemcpyAsync(m->res_halo.get(), list.data(), list.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                              st));
+    FK_HIP(hipStreamSynchronize(st));
+    m->res_R = R;
+    m->res_width = most;
+    m->res_halo_max = hmax;
+}
+
+// the copy of the matrix a resident launch can run on, with fresh values
+static bool resident_kind(const fk_mesh *m) {
+    if (m->ctx->timing.enabled) return false;
+    if (m->kind == FK_SPMV_STENCIL) return m->st_K <= kResK;
+    return m->kind == FK_SPMV_SELL64 && m->format != FK_SPMV_CSR && m->have_sell && m->res_R > 0;
+}
+
 bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, CgState *out) {
-    if (m->kind != FK_SPMV_STENCIL || m->st_K > kResK || m->ctx->timing.enabled) return false;
+    if (!resident_kind(m)) return false;
+    const bool stencil = m->kind == FK_SPMV_STENCIL;
     PcgWork<double> &w = m->w64;
     ResidentArgs<double> A{};
-    A.val = m->st_val64.get();
+    A.val = stencil ? m->st_val64.get() : m->sell_val64.get();
     A.dinv = w.dinv.get();
     A.r0 = w.r.get();
     A.x = w.x.get();
@@ -585,7 +818,7 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
     // one resident launch of this process at a time on the device: the blocks
     // of two would take each other's CUs and wait for blocks not yet started
     const std::lock_guard<std::mutex> alone(resident_mutex(m->ctx->device));
-    if (!launch_by_rows(m, A)) return false;
+    if (!(stencil ? launch_by_rows(m, A) : launch_sell(m, A))) return false;
     hipStream_t st = m->ctx->stream;
     CgState *hs = m->hstate.ptr;
     FK_HIP(hipMemcpyAsync(hs, w.state.get(), sizeof(CgState), hipMemcpyDeviceToHost, st));
@@ -600,14 +833,15 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
 // allow a resident launch; u and r64 may then have changed.
 bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
                       int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status) {
-    if (m->kind != FK_SPMV_STENCIL || m->st_K > kResK || m->ctx->timing.enabled) return false;
+    if (!resident_kind(m)) return false;
+    const bool stencil = m->kind == FK_SPMV_STENCIL;
     PcgWork<float> &w = m->w32;
     if (!m->ru) {
         m->ru.alloc(1);
         m->hru.alloc(2);
     }
     ResidentArgs<float> A{};
-    A.val = m->st_val32.get();
+    A.val = stencil ? m->st_val32.get() : m->sell_val32.get();
     A.dinv = w.dinv.get();
     A.state = w.state.get();
     A.ld = static_cast<int32_t>(m->st_ld);
@@ -617,7 +851,7 @@ bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double 
     A.u = u;
     A.b = b;
     A.r64 = m->r64.get();
-    A.val64 = m->st_val64.get();
+    A.val64 = stencil ? m->st_val64.get() : m->sell_val64.get();
     A.diag64 = m->sell_diag64.get();
     A.ru = m->ru.get();
     A.p = w.p.get();
@@ -627,7 +861,7 @@ bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double 
     A.delta2 = delta * delta;
     A.G = chunk;
     const std::lock_guard<std::mutex> alone(resident_mutex(m->ctx->device));
-    if (!launch_by_rows(m, A)) return false;
+    if (!(stencil ? launch_by_rows(m, A) : launch_sell(m, A))) return false;
     hipStream_t st = m->ctx->stream;
     CgState *hs = m->hstate.ptr;
     RuState *hr = m->hru.ptr;

@@ -1254,6 +1254,7 @@ static void build_sell(fk_mesh *m) {
     if (len > 0)
         FK_HIP(hipMemcpyAsync(m->sell_map.get(), map.data(), len * sizeof(int32_t), hipMemcpyHostToDevice, st));
     FK_HIP(hipStreamSynchronize(st));  // host vectors go out of scope
+    build_resident_sell(m, rp, ci, width, shared, vptr);
     m->have_sell = true;
 }
 

@@ -111,6 +111,41 @@ def test_right_hand_sides(contexts, n, precision):
     _increment(contexts, n, precision)
 
 
+# a mesh generator's numbering: the SELL copy of the renumbered mesh, at the
+# edges of its launch shapes (512, 1024, 1536, 2048 rows per block)
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("n", [3, 8, 20, 49, 50, 63, 64, 72, 73, 79, 80])
+def test_scattered_numbering(contexts, n, precision):
+    pr = W.linear(n)
+    pr = W.renumbered(pr, np.random.default_rng(n).permutation(pr.mesh.nv), "scattered")
+    order = np.random.default_rng(n + 1).permutation(pr.mesh.nt)
+    mesh = MESH(p=pr.mesh.p, t=np.asfortranarray(pr.mesh.t[:, order]), VE=pr.mesh.VE[order])
+    _both(contexts, mesh, pr.mu[order], pr.mask, pr.g, precision=precision)
+
+
+# Delaunay meshes: rows of 4 to over 30 entries (beyond 32: the three kernels)
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("points", [60, 700, 9000])
+def test_delaunay(contexts, points, precision):
+    from scipy.spatial import Delaunay
+
+    rng = np.random.default_rng(points)
+    pts = np.concatenate([rng.random((points, 3)), np.array([[i, j, k] for i in (0, 1) for j in (0, 1)
+                                                             for k in (0, 1)], float)])
+    tri = Delaunay(pts, qhull_options="QJ").simplices
+    p = np.asfortranarray(pts.T)
+    t = np.asfortranarray((tri.T + 1).astype(np.int32))
+    vol = element_volumes(p, t)
+    t = np.asfortranarray(t[:, vol > 1e-9])
+    mesh = MESH(p=p, t=t, VE=element_volumes(p, t))
+    used = np.zeros(mesh.nv, bool)
+    used[t.ravel() - 1] = True
+    mask = (~used) | (p[2] < 0.15) | (p[2] > 0.85)
+    g = np.where(mask, p[2], 0.0)
+    mu = MU0 * rng.uniform(1.0, 20.0, mesh.nt)
+    _both(contexts, mesh, mu, mask.astype(np.uint8), g, precision=precision)
+
+
 # one cell thick (too much padding for the stencil copy: SELL), long columns,
 # flat plates: one merged window, split windows, and offsets too far apart for
 # three windows (the three-kernel iteration on both)
