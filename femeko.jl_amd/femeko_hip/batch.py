@@ -9,7 +9,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import FemekoHIPError, dptr, iptr, uptr
-from .device import Context, context
+from .device import Context, _live_meshes, context
 
 
 @dataclass
@@ -39,6 +39,7 @@ class Batch:
                                     ctypes.byref(h))
         self.ctx.check(s, "fk_batch_create")
         self.handle = h
+        _live_meshes.add(self)
         self._p = self._t = None
         nodes = ctypes.c_int64(0)
         nnz = ctypes.c_int64(0)

@@ -73,7 +73,7 @@ _live_meshes = weakref.WeakSet()
 
 @atexit.register
 def _release_all():
-    # free device memory while the HIP runtime is still up: meshes, then contexts
+    # free device memory while the HIP runtime is still up: meshes and batches, then contexts
     for dm in list(_live_meshes):
         dm.close()
     for ctx in list(_default.values()):

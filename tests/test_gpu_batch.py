@@ -246,3 +246,14 @@ def test_batch_other_field_counts(oracle, nrhs, fmt):
                 assert err < 1e-9, (nrhs, fmt, i, j, err)
     finally:
         b.close()
+
+
+def test_batch_is_released_with_its_context():
+    """An open batch is closed before the context at interpreter exit."""
+    from femeko_hip import device
+
+    probs = small_batch(count=1)
+    b = Batch([probs[0].mesh], nrhs=1)
+    assert any(x is b for x in device._live_meshes)
+    b.close()
+    b.close()
