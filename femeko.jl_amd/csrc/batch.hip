@@ -82,6 +82,9 @@ struct fk_batch {
     fk::DevBuf<int64_t> st_vbase;
     fk::DevBuf<float> st_val32;
     fk::DevBuf<double> st_val64, st_diag64;  // FP64 copy and diagonal for the true residuals
+    std::vector<int32_t> h_off, h_K;         // the meshes' offsets (16 each) and their counts
+    std::vector<int64_t> h_vbase;
+    fk::ResidentBatch res;                   // resident launches (resident.hip)
     ~fk_batch() {
         if (graph) (void)hipGraphExecDestroy(graph);
         if (ru_graph) (void)hipGraphExecDestroy(ru_graph);
@@ -1351,33 +1354,74 @@ static void enqueue_ru_chunk(fk_batch *b, const BatchRu &u, int G) {
     FK_HIP(hipGetLastError());
 }
 
-// FP32 PCG per system with FP64 reliable updates decided on the device
-static void batch_solve_ru(fk_batch *b, double rtol, double delta, int64_t max_iter, int64_t *iters_out,
-                           int32_t *outer_out, double *relres_out) {
+// The systems still to be solved, on resident launches; false: not for this
+// batch, r64 and phi then need a fresh start.
+static bool batch_solve_resident(fk_batch *b, double delta, int64_t max_iter, const std::vector<int32_t> &act,
+                                 const std::vector<double> &scale, const std::vector<double> &th,
+                                 const std::vector<double> &t2, std::vector<int64_t> &its, std::vector<int32_t> &nrep,
+                                 std::vector<int32_t> &fst, std::vector<double> &rr64) {
+    if (b->ctx->timing.enabled || b->stencil != 1 || !b->st_valid) return false;
+    fk_mesh *m = b->mesh;
+    const int nr = b->nrhs;
+    std::vector<ResidentSystem> sys;
+    std::vector<int> which;
+    for (int q = 0; q < b->nmesh; ++q)
+        for (int j = 0; j < nr; ++j) {
+            const int s = q * nr + j;
+            if (!act[s]) continue;
+            const int64_t a = b->node_off[q], n = b->node_off[q + 1] - a;
+            if (n * nr >= (int64_t(1) << 28)) return false;
+            ResidentSystem y{};
+            y.val32 = b->st_val32.get() + b->h_vbase[q];
+            y.val64 = b->st_val64.get() + b->h_vbase[q];
+            y.diag64 = b->st_diag64.get() + a;
+            y.dinv = m->w32.dinv.get() + a;
+            y.n = static_cast<int32_t>(n);
+            y.K = b->h_K[q];
+            y.off = b->h_off.data() + 16 * q;
+            y.us = nr;
+            y.u = b->phi.get() + a * nr + j;
+            y.r64 = b->r64.get() + a * nr + j;
+            y.p = b->p.get() + a * nr + j * n;
+            y.s = 1.0 / scale[s];
+            y.target2 = t2[s];
+            y.thresh64 = th[s];
+            sys.push_back(y);
+            which.push_back(s);
+        }
+    std::vector<CgState> state;
+    std::vector<RuState> ru;
+    b->res.ctx = b->ctx;
+    if (!resident_batch(b->res, sys, delta, max_iter, 16, state, ru)) {
+        if (b->res.started) {  // timed out: back to the start
+            kb_init_phi<<<grid_for(m->nv * nr, 256), 256, 0, b->ctx->stream>>>(b->phi.get(), b->g.get(), m->mask.get(),
+                                                                               m->nv, nr);
+            FK_HIP(hipGetLastError());
+            neg_residual_batch(b, b->phi.get());
+        }
+        return false;
+    }
+    for (size_t k = 0; k < sys.size(); ++k) {
+        its[which[k]] = state[k].iters;
+        nrep[which[k]] = ru[k].nrep;
+        fst[which[k]] = ru[k].status;
+        rr64[which[k]] = ru[k].rr64;
+    }
+    return true;
+}
+
+// The same in chunks of iterations (three kernels each) and replacement steps,
+// captured once in a graph.
+static void batch_solve_chunks(fk_batch *b, double delta, int64_t max_iter, const std::vector<int32_t> &act,
+                               const std::vector<double> &rr, std::vector<int64_t> &its, std::vector<int32_t> &nrep,
+                               std::vector<int32_t> &fst, std::vector<double> &rr64, const std::vector<double> &th,
+                               const std::vector<double> &scale, const std::vector<double> &t2) {
     fk_mesh *m = b->mesh;
     hipStream_t st = b->ctx->stream;
-    const int64_t nv = m->nv;
-    const int nr = b->nrhs, S = b->nsys;
-    b->phi.ensure(nv * nr);
-    b->r64.ensure(nv * nr);
-    kb_init_phi<<<grid_for(nv * nr, 256), 256, 0, st>>>(b->phi.get(), b->g.get(), m->mask.get(), nv, nr);
-    b->have_phi = true;
-    std::vector<double> bb, rr;
-    neg_residual_batch(b, b->g.get());  // b = -A[free,fixed] g per system
-    system_norms(b, bb);
-    neg_residual_batch(b, b->phi.get());  // r64 = residual of the start
-    system_norms(b, rr);
-    std::vector<int32_t> act(S), fin(S);
-    std::vector<double> scale(S), th(S), t2(S);
-    int nfin0 = 0;
-    for (int s = 0; s < S; ++s) {
-        th[s] = rtol * rtol * bb[s];
-        act[s] = (bb[s] > 0.0 && !(rr[s] < th[s])) ? 1 : 0;
-        fin[s] = !act[s];
-        nfin0 += fin[s];
-        scale[s] = act[s] ? std::sqrt(rr[s]) : 1.0;
-        t2[s] = act[s] ? th[s] / rr[s] : 0.0;
-    }
+    const int S = b->nsys;
+    std::vector<int32_t> fin(S);
+    int32_t nfin0 = 0;
+    for (int s = 0; s < S; ++s) nfin0 += fin[s] = !act[s];
     DevBuf<double> target2(S);
     std::vector<int32_t> zeros(S, 0);
     FK_HIP(hipMemcpyAsync(b->active.get(), act.data(), S * sizeof(int32_t), hipMemcpyHostToDevice, st));
@@ -1437,14 +1481,43 @@ static void batch_solve_ru(fk_batch *b, double rtol, double delta, int64_t max_i
     }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
-    std::vector<int64_t> its(S);
-    std::vector<int32_t> nrep(S), fst(S);
-    std::vector<double> rr64(S);
     FK_HIP(hipMemcpyAsync(its.data(), b->iters.get(), S * sizeof(int64_t), hipMemcpyDeviceToHost, st));
     FK_HIP(hipMemcpyAsync(nrep.data(), b->ru_nrep.get(), S * sizeof(int32_t), hipMemcpyDeviceToHost, st));
     FK_HIP(hipMemcpyAsync(fst.data(), b->ru_status.get(), S * sizeof(int32_t), hipMemcpyDeviceToHost, st));
     FK_HIP(hipMemcpyAsync(rr64.data(), b->rr64.get(), S * sizeof(double), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
+}
+
+// FP32 PCG per system with FP64 reliable updates decided on the device
+static void batch_solve_ru(fk_batch *b, double rtol, double delta, int64_t max_iter, int64_t *iters_out,
+                           int32_t *outer_out, double *relres_out) {
+    fk_mesh *m = b->mesh;
+    hipStream_t st = b->ctx->stream;
+    const int64_t nv = m->nv;
+    const int nr = b->nrhs, S = b->nsys;
+    b->phi.ensure(nv * nr);
+    b->r64.ensure(nv * nr);
+    kb_init_phi<<<grid_for(nv * nr, 256), 256, 0, st>>>(b->phi.get(), b->g.get(), m->mask.get(), nv, nr);
+    b->have_phi = true;
+    std::vector<double> bb, rr;
+    neg_residual_batch(b, b->g.get());  // b = -A[free,fixed] g per system
+    system_norms(b, bb);
+    neg_residual_batch(b, b->phi.get());  // r64 = residual of the start
+    system_norms(b, rr);
+    std::vector<int32_t> act(S);
+    std::vector<double> scale(S), th(S), t2(S);
+    for (int s = 0; s < S; ++s) {
+        th[s] = rtol * rtol * bb[s];
+        act[s] = (bb[s] > 0.0 && !(rr[s] < th[s])) ? 1 : 0;
+        scale[s] = act[s] ? std::sqrt(rr[s]) : 1.0;
+        t2[s] = act[s] ? th[s] / rr[s] : 0.0;
+    }
+    std::vector<int64_t> its(S, 0);
+    std::vector<int32_t> nrep(S, 0), fst(S, FK_OK);
+    std::vector<double> rr64(rr);
+    if (!batch_solve_resident(b, delta, max_iter, act, scale, th, t2, its, nrep, fst, rr64)) {
+        batch_solve_chunks(b, delta, max_iter, act, rr, its, nrep, fst, rr64, th, scale, t2);
+    }
     int status = FK_OK;
     for (int s = 0; s < S; ++s) {
         if (iters_out) iters_out[s] = act[s] ? its[s] : 0;
@@ -1581,6 +1654,9 @@ static void build_batch_stencil(fk_batch *b) {
                           hipMemcpyHostToDevice, st));
     FK_HIP(hipStreamSynchronize(st));
     build_spmm_table(b);
+    b->h_off = offs;
+    b->h_K = K;
+    b->h_vbase = vbase;
     b->st_len = len;
     b->st_Kc = K[0];
     for (int q = 1; q < M; ++q)

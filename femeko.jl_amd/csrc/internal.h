@@ -352,6 +352,31 @@ CgState run_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref);
 int solve_f32_increment(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, int64_t *iters);
 int solve_f32_free(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, double bb_ref,
                    int64_t *iters, double *rr_out, double *bb_out);
+// one system of a batch: the stencil copy of its mesh (columns of n rows), its
+// potential and residual (a row's values us apart), scratch p of n values
+struct ResidentSystem {
+    const float *val32, *dinv;
+    const double *val64, *diag64;
+    int32_t n, K, us;
+    const int32_t *off;               // host
+    double *u, *r64;
+    float *p;
+    double s, target2, thresh64;      // residual scale, scaled and FP64 target of ||r||^2
+};
+struct ResidentBatch {
+    fk_context *ctx = nullptr;
+    bool started = false;  // the last call changed u and r64
+    DevBuf<unsigned long long> words;
+    DevBuf<float> w;
+    DevBuf<char> args;
+    DevBuf<int2> table;
+    DevBuf<CgState> state;
+    DevBuf<RuState> ru;
+};
+// FP32-refined solves of all systems in cooperative launches (resident.hip);
+// false: not for this batch, or a wait timed out (started)
+bool resident_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sys, double delta, int64_t max_iter, int chunk,
+                    std::vector<CgState> &state, std::vector<RuState> &ru);
 struct NeumannResult {
     double multiplier;
     int64_t iters;

@@ -87,16 +87,16 @@ constexpr int kMaxResidentBlocks = 256;
 constexpr int kReduceCopies = 8;
 constexpr int kReduceLine = 16;   // words of a line, ten used
 constexpr int kReduceWaves = 8;   // polling waves of a block
-constexpr int kReduceWords = 2 * kReduceCopies * kMaxResidentBlocks * kReduceLine;
+constexpr int reduce_words(int nb) { return 2 * kReduceCopies * nb * kReduceLine; }
 constexpr int kReduceShared = 5 * 16 + 5 * kReduceWaves + 1;  // doubles of LDS
 
-// Sum of v[0..5) over all threads of all blocks, the same bits in every
-// thread; false when the wait ran out. Before the blocks' partials leave, every
+// Sum of v[0..5) over all threads of the nb blocks of a group (block `me` of
+// it), the same bits in every thread; false when the wait ran out. Before the blocks' partials leave, every
 // wave waits for its earlier stores, so agent-scope stores made before the
 // call are visible to agent-scope loads made after it. sh: kReduceShared
-// doubles, the last one 0 before the first call; lines: kReduceWords words.
+// doubles, the last one 0 before the first call; lines: reduce_words(nb) words.
 template <int BLOCK>
-__device__ __forceinline__ bool all_reduce5(double (&v)[5], u64 *__restrict__ lines, int nb, uint32_t tag,
+__device__ __forceinline__ bool all_reduce5(double (&v)[5], u64 *__restrict__ lines, int me, int nb, uint32_t tag,
                                             double *sh) {
     constexpr int W = BLOCK / 64, P = kReduceWaves;
     static_assert(W >= P && W <= 16, "one row of lanes adds the wave sums");
@@ -108,14 +108,14 @@ __device__ __forceinline__ bool all_reduce5(double (&v)[5], u64 *__restrict__ li
     if (l == 0) sh[4 * 16 + w] = f4;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    u64 *base = lines + (tag & 1) * (kReduceWords / 2);
+    u64 *base = lines + (tag & 1) * (kReduceCopies * kReduceLine * nb);
     if (w == 0) {
         // lane 16 k + 2 copy + half writes that half of value k
         const u64 a = static_cast<u64>(__double_as_longlong(row16_sum(c < W ? sh[row * 16 + c] : 0.0)));
         const u64 b = static_cast<u64>(__double_as_longlong(row16_sum(c < W ? sh[4 * 16 + c] : 0.0)));
         const int copy = c >> 1, half = c & 1;
         static_assert(kReduceCopies == 8, "16 lanes write two halves to each copy");
-        u64 *line = base + (copy * kMaxResidentBlocks + blockIdx.x) * kReduceLine;
+        u64 *line = base + (copy * nb + me) * kReduceLine;
         const u64 high = 0xffffffff00000000ull;
         __hip_atomic_store(line + 2 * row + half, (half ? a & high : a << 32) | tag, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
@@ -125,7 +125,7 @@ __device__ __forceinline__ bool all_reduce5(double (&v)[5], u64 *__restrict__ li
     }
     if (w < P) {
         // a row of lanes polls a line; block 4 P i + 4 w + row
-        const u64 *mine = base + (blockIdx.x % kReduceCopies) * (kMaxResidentBlocks * kReduceLine);
+        const u64 *mine = base + (me % kReduceCopies) * (nb * kReduceLine);
         constexpr int PER = kMaxResidentBlocks / (4 * P);
         u64 a[PER];
 #pragma unroll

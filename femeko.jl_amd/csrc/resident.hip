@@ -72,6 +72,7 @@ struct ResidentArgs {
     const double *val64, *diag64;
     T *p;                         // the direction of the own rows over a replacement
     RuState *ru;
+    int32_t us;                   // distance of a row's values in u and r64 (right-hand sides side by side)
     double s, target2, thresh64, delta2;
     int32_t G;                    // iterations between two checks of the drop
 };
@@ -86,12 +87,12 @@ __device__ __forceinline__ int32_t fresh(int32_t v) {
 
 // LDS index of the e-th window element (the windows in LDS order, the own rows
 // left out; elements past the last share one spare slot) and its row (spare: none)
-template <typename T>
-__device__ __forceinline__ int32_t window_lds(const ResidentArgs<T> &A, int32_t R, int32_t e) {
+template <typename Args>
+__device__ __forceinline__ int32_t window_lds(Args &A, int32_t R, int32_t e) {
     return min(e < A.lown ? e : e + R, A.wbeg[kResWindows]);
 }
-template <typename T>
-__device__ __forceinline__ int32_t window_row(const ResidentArgs<T> &A, int32_t i0, int32_t li) {
+template <typename Args>
+__device__ __forceinline__ int32_t window_row(Args &A, int32_t i0, int32_t li) {
     int32_t d = A.wrow[0];
 #pragma unroll
     for (int k = 1; k < kResWindows; ++k) d = li >= A.wbeg[k] ? A.wrow[k] : d;
@@ -120,8 +121,8 @@ constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursio
 // rows replaces the recursion's (times s), and p is kept; a recursion that has
 // drifted below the true residual, or broken down, restarts from p = z. The
 // solve ends on the FP64 residual.
-template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE, int NE>
-__global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A) {
+template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE, int NE, typename Args>
+__device__ __forceinline__ void resident_solve(Args &A, const int me, const int32_t i0) {
     extern __shared__ char lds_raw[];
     T *win = reinterpret_cast<T *>(lds_raw);
     __shared__ double sh[kReduceShared];
@@ -133,7 +134,6 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
     constexpr bool XLDS = x_in_lds<T>(RPT);
     T *xs = win + (GEN ? A.spare : A.wbeg[kResWindows]) + 1;
     constexpr bool AHEAD = RPT > 1 && (sizeof(T) == 4 || (!GEN && RPT <= 3));
-    const int32_t i0 = logical_block(A.nb) * R;
     const int32_t tid = threadIdx.x;
     const AgentRows<T> rows(A.w, A.stride);
     const ValueColumns<T> vals(A.val, A.K, A.ld);
@@ -151,10 +151,10 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
         if (row >= n) continue;
         const T dj = A.dinv[row];
         T r = T(0);
-        if (dj != T(0)) r = REFINE ? static_cast<T>(A.s * A.r64[row]) : A.r0[row];
+        if (dj != T(0)) r = REFINE ? static_cast<T>(A.s * A.r64[static_cast<int64_t>(row) * A.us]) : A.r0[row];
         rows.store(tag, row, dj * r);
     }
-    bool alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+    bool alive = all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
 
     double rr = 0.0, thresh = 0.0, bb = A.bb_ref;
     int64_t it = 0;
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                 s[4] += rd * rd;
                 __builtin_amdgcn_sched_barrier(0);
             }
-            alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+            alive = all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
             T ww[U];
             const int32_t ft = fresh(tid);
 #pragma unroll
@@ -380,20 +380,21 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
             }
             restart = act == 2;
             const int32_t tc = fresh(tid);
-            const AgentRows<double> sol(A.u, n);
+            const AgentRows<double> sol(A.u, n * A.us);
+            const auto at = [&](int32_t row) { return static_cast<int64_t>(row) * A.us; };
             if (act == 1) {
                 const double inv_s = 1.0 / A.s;
 #pragma unroll
                 for (int j = 0; j < RPT; ++j) {
                     const int32_t row = i0 + j * BLOCK + tc;
                     if (row < n) {
-                        sol.store(0, row, A.u[row] + inv_s * static_cast<double>(x[XLDS ? 0 : j]));
+                        sol.store(0, row * A.us, A.u[at(row)] + inv_s * static_cast<double>(x[XLDS ? 0 : j]));
                         A.p[row] = p[j];
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 ++tag;
-                alive = all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+                alive = all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
                 // the other blocks' u through this CU's caches: one wave's
                 // acquire serves the block (a fence in every wave takes 16
                 // times as long)
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                 const int32_t row = i0 + j * BLOCK + tc;
                 if (row >= n) continue;
                 const T dj = A.dinv[row];
-                double v = dj != T(0) ? A.r64[row] : 0.0;
+                double v = dj != T(0) ? A.r64[at(row)] : 0.0;
                 if (act == 1) {
                     double y0 = 0.0, y1 = 0.0;
                     if constexpr (GEN) {
@@ -422,10 +423,10 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                         const int32_t W = abs(A.swidth[sl]), ng = W >> 2;
 #pragma unroll 4
                         for (int k = 0; k < W; ++k) {
-                            const int64_t at = base + (k < 4 * ng ? 4 * (64 * (k >> 2) + lane) + (k & 3)
-                                                                  : 256 * ng + 64 * (k - 4 * ng) + lane);
-                            const int32_t ix = A.sidx[at];
-                            y0 += A.val64[at] * A.u[ix < R ? i0 + ix : A.halo[h0 + ix - R]];
+                            const int64_t e = base + (k < 4 * ng ? 4 * (64 * (k >> 2) + lane) + (k & 3)
+                                                                 : 256 * ng + 64 * (k - 4 * ng) + lane);
+                            const int32_t ix = A.sidx[e];
+                            y0 += A.val64[e] * A.u[at(ix < R ? i0 + ix : A.halo[h0 + ix - R])];
                         }
                     } else {
 #pragma unroll
@@ -434,18 +435,18 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
                                 const int32_t o = A.off[k], f = min(row + o, n - 1), bk = max(row - o, 0);
                                 const double *__restrict__ c = A.val64 + static_cast<int64_t>(k) * A.ld;
                                 const double vb64 = c[bk];
-                                y0 += c[row] * A.u[f];  // 0 where row + o is past the last row
-                                y1 += (row >= o ? vb64 : 0.0) * A.u[bk];
+                                y0 += c[row] * A.u[at(f)];  // 0 where row + o is past the last row
+                                y1 += (row >= o ? vb64 : 0.0) * A.u[at(bk)];
                             }
                     }
-                    const double y = (y0 + y1) + A.diag64[row] * A.u[row];
+                    const double y = (y0 + y1) + A.diag64[row] * A.u[at(row)];
                     v = dj != T(0) ? (A.b ? A.b[row] - y : -y) : 0.0;
-                    A.r64[row] = v;
+                    A.r64[at(row)] = v;
                     s[0] += v * v;
                 }
                 rows.store(tag, row, dj * static_cast<T>(A.s * v));
             }
-            alive = alive && all_reduce5<BLOCK>(s, A.slots, A.nb, tag, sh);
+            alive = alive && all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
             if (!alive) {
                 code = FK_ERR_HIP;
                 break;
@@ -465,7 +466,7 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
             }
         }
     }
-    if (blockIdx.x == 0 && tid == 0) {
+    if (me == 0 && tid == 0) {
         if constexpr (REFINE) {
             A.ru->nrep = nrep;
             A.ru->restarts = restarts;
@@ -481,6 +482,24 @@ __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A)
     }
 }
 
+template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE, int NE>
+__global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A) {
+    resident_solve<T, BLOCK, RPT, NK, U, REFINE, NE>(A, static_cast<int>(blockIdx.x),
+                                                     logical_block(A.nb) * (BLOCK * RPT));
+}
+
+// Several systems in one launch: block b is block first[b].y of system
+// first[b].x. The arguments are read as constants, as kernel arguments are.
+template <typename T, int BLOCK, int RPT, int NK, int U>
+__global__ __launch_bounds__(BLOCK) void k_resident_batch(const ResidentArgs<T> *__restrict__ all,
+                                                          const int2 *__restrict__ first) {
+    using Const = const __attribute__((address_space(4))) ResidentArgs<T>;
+    const int2 b = first[blockIdx.x];
+    const int sys = __builtin_amdgcn_readfirstlane(b.x), me = __builtin_amdgcn_readfirstlane(b.y);
+    Const &A = *((Const *)(all + sys));
+    resident_solve<T, BLOCK, RPT, NK, U, true, 0>(A, me, me * (BLOCK * RPT));
+}
+
 // slots, and the rows n..stride of the two exchange arrays
 template <typename T>
 __global__ void k_resident_clear(u64 *__restrict__ slots, int words, T *__restrict__ w, int32_t n, int32_t stride) {
@@ -489,17 +508,23 @@ __global__ void k_resident_clear(u64 *__restrict__ slots, int words, T *__restri
     for (int i = n + t; i < stride; i += step) w[i] = w[stride + i] = T(0);
 }
 
+__global__ void k_resident_zero(u64 *__restrict__ a, int64_t na, float *__restrict__ b, int64_t nb) {
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    for (int64_t i = t; i < na; i += step) a[i] = 0;
+    for (int64_t i = t; i < nb; i += step) b[i] = 0.f;
+}
+
 // ---------------------------------------------------------------------------
 // host side
 
 // The windows of a block of R rows, in LDS one after another. False when they
 // are too many or too long.
 template <typename T>
-static bool place_windows(const fk_mesh *m, int R, ResidentArgs<T> &A, int32_t *elements) {
-    const int K = m->st_K;
+static bool place_windows(const int32_t *off, int K, int R, ResidentArgs<T> &A, int32_t *elements) {
     std::vector<std::pair<int64_t, int64_t>> iv{{0, R}};
     for (int k = 0; k < K; ++k) {
-        const int64_t o = m->st_off[k];
+        const int64_t o = off[k];
         iv.push_back({o, o + R});
         iv.push_back({-o, R - o});
     }
@@ -528,7 +553,7 @@ static bool place_windows(const fk_mesh *m, int R, ResidentArgs<T> &A, int32_t *
     };
     A.lown = place(0);
     for (int k = 0; k < kResK; ++k) {
-        A.off[k] = k < K ? m->st_off[k] : 0;
+        A.off[k] = k < K ? off[k] : 0;
         A.lf[k] = place(A.off[k]);
         A.lb[k] = place(-static_cast<int64_t>(A.off[k]));
     }
@@ -555,7 +580,7 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
         A.halo = m->res_halo.get();
         A.nslices = static_cast<int32_t>(m->nslices);
     } else {
-        if (!place_windows<T>(m, R, A, &elements) || elements - R > U * BLOCK) return false;
+        if (!place_windows<T>(m->st_off, m->st_K, R, A, &elements) || elements - R > U * BLOCK) return false;
     }
     const size_t lds = (static_cast<size_t>(elements) + 1 + (x_in_lds<T>(RPT) ? R : 0)) * sizeof(T);
     if (lds > static_cast<size_t>(kResLdsMax)) return false;
@@ -564,7 +589,7 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     const int64_t reach = static_cast<int64_t>(nb) * R + (NE > 0 ? 0 : m->st_off[m->st_K - 1] + R);
     const int64_t stride = (reach + 63) / 64 * 64;
     hipStream_t st = m->ctx->stream;
-    m->res_slots.ensure(kReduceWords);
+    m->res_slots.ensure(reduce_words(kMaxResidentBlocks));
     m->res_w.ensure(static_cast<size_t>(2 * stride));
     A.stride = static_cast<int32_t>(stride);
     A.slots = m->res_slots.get();
@@ -572,7 +597,7 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     auto kern = k_resident_pcg<T, BLOCK, RPT, NK, U, REFINE, NE>;
     FK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                static_cast<int>(lds)));
-    k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, kReduceWords, A.w, A.n, A.stride);
+    k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, reduce_words(nb), A.w, A.n, A.stride);
     FK_HIP(hipGetLastError());
     void *args[] = {&A};
     const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kern), dim3(nb), dim3(BLOCK),
@@ -855,6 +880,7 @@ bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double 
     A.diag64 = m->sell_diag64.get();
     A.ru = m->ru.get();
     A.p = w.p.get();
+    A.us = 1;
     A.s = 1.0 / std::sqrt(rr);
     A.target2 = thresh * A.s * A.s;
     A.thresh64 = thresh;
@@ -873,6 +899,151 @@ bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double 
     *nrep = hr->nrep;
     *rr_out = hr->rr64;
     *status = hr->status;
+    return true;
+}
+
+// ---- batches ----------------------------------------------------------------
+// Every system (mesh, right-hand side) is a group of blocks of its own that
+// solves and stops by itself; a launch holds as many systems as fit the chip at
+// once, so no group ever waits for a block that has not started. Systems are
+// packed into launches largest first: those of one launch take about equally
+// many iterations.
+//
+// Rows per block: the fewest with which one launch holds the batch (an
+// iteration takes 4.6, 5.2 and 6.2 us with 512, 1024 and 2048 rows a block),
+// else 2048, and no more than kResBatchLaunches launches: a launch ends with
+// its slowest system, and with many of them the three kernels per iteration,
+// which read a matrix value once for all right-hand sides of its mesh, win.
+// Solve of 3 right-hand sides per mesh, three kernels against launches of 2048
+// rows a block: 10 meshes of 10..20 cells 3.89 to 1.05 ms (0.80 with 512 rows),
+// 20 of 10..40 (3 launches) 15.5 to 5.4, 6 of 40..50 (4) 19.6 to 10.2, 40 of
+// 10..44 (7) 21.7 to 14.6, 50 of 10..50 (12) 36.1 to 29.3, 100 of 10..40 (15)
+// 30.1 to 28.0, 16 of 50..60 (17) 55.4 to 65.2, 64 of 10..60 (27) 67.1 to 71.3.
+constexpr size_t kResBatchLaunches = 12;
+
+template <int BLOCK, int RPT, int NK>
+static bool launch_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sys, double delta, int64_t max_iter,
+                         int chunk, size_t most) {
+    constexpr int R = BLOCK * RPT, U = 2 * RPT + 2;
+    if (B.started) return false;  // an earlier shape did not fit the device after all
+    fk_context *ctx = B.ctx;
+    hipStream_t st = ctx->stream;
+    const int S = static_cast<int>(sys.size());
+    std::vector<ResidentArgs<float>> args(static_cast<size_t>(S));
+    size_t lds = 0;
+    int64_t words = 0, floats = 0;
+    for (int s = 0; s < S; ++s) {
+        const ResidentSystem &q = sys[s];
+        ResidentArgs<float> &A = args[s];
+        int32_t elements = 0;
+        if (q.K < 1 || q.K > kResK || !place_windows<float>(q.off, q.K, R, A, &elements) || elements - R > U * BLOCK) return false;
+        lds = std::max(lds, (static_cast<size_t>(elements) + 1) * sizeof(float));
+        A.nb = (q.n + R - 1) / R;
+        if (A.nb > kMaxResidentBlocks) return false;
+        A.stride = static_cast<int32_t>((static_cast<int64_t>(A.nb) * R + q.off[q.K - 1] + R + 63) / 64 * 64);
+        words += reduce_words(A.nb);
+        floats += 2 * static_cast<int64_t>(A.stride);
+    }
+    if (lds > static_cast<size_t>(kResLdsMax)) return false;
+    auto kern = k_resident_batch<float, BLOCK, RPT, NK, U>;
+    FK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               static_cast<int>(lds)));
+    int per_cu = 0;
+    FK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kern), BLOCK, lds));
+    const int room = std::min(per_cu, 2) * ctx->num_cus;
+    if (room < 1) return false;
+    for (const ResidentArgs<float> &A : args)
+        if (A.nb > room) return false;
+    // launches: first fit, largest systems first
+    std::vector<int> order(static_cast<size_t>(S));
+    for (int s = 0; s < S; ++s) order[s] = s;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sys[a].n > sys[b].n; });
+    std::vector<std::vector<int2>> rounds;
+    for (int s : order) {
+        size_t k = 0;
+        while (k < rounds.size() && static_cast<int>(rounds[k].size()) + args[s].nb > room) ++k;
+        if (k == rounds.size()) rounds.emplace_back();
+        for (int b = 0; b < args[s].nb; ++b) rounds[k].push_back(make_int2(s, b));
+    }
+    if (rounds.size() > most) return false;
+    B.words.ensure(words);
+    B.w.ensure(floats);
+    B.args.ensure(S * sizeof(ResidentArgs<float>));
+    B.state.ensure(S);
+    B.ru.ensure(S);
+    words = floats = 0;
+    for (int s = 0; s < S; ++s) {
+        const ResidentSystem &q = sys[s];
+        ResidentArgs<float> &A = args[s];
+        A.val = q.val32;
+        A.dinv = q.dinv;
+        A.w = B.w.get() + floats;
+        A.slots = B.words.get() + words;
+        A.state = B.state.get() + s;
+        A.ld = q.n;
+        A.n = q.n;
+        A.K = q.K;
+        A.max_iter = max_iter;
+        A.u = q.u;
+        A.us = q.us;
+        A.r64 = q.r64;
+        A.val64 = q.val64;
+        A.diag64 = q.diag64;
+        A.p = q.p;
+        A.ru = B.ru.get() + s;
+        A.s = q.s;
+        A.target2 = q.target2;
+        A.thresh64 = q.thresh64;
+        A.delta2 = delta * delta;
+        A.G = chunk;
+        words += reduce_words(A.nb);
+        floats += 2 * static_cast<int64_t>(A.stride);
+    }
+    std::vector<int2> table;
+    for (const auto &r : rounds) table.insert(table.end(), r.begin(), r.end());
+    B.table.ensure(table.size());
+    FK_HIP(hipMemcpyAsync(B.args.get(), args.data(), S * sizeof(ResidentArgs<float>), hipMemcpyHostToDevice, st));
+    FK_HIP(hipMemcpyAsync(B.table.get(), table.data(), table.size() * sizeof(int2), hipMemcpyHostToDevice, st));
+    k_resident_zero<<<256, 256, 0, st>>>(B.words.get(), words, B.w.get(), floats);
+    FK_HIP(hipGetLastError());
+    const auto *dargs = reinterpret_cast<const ResidentArgs<float> *>(B.args.get());
+    const int2 *at = B.table.get();
+    B.started = true;
+    for (const auto &r : rounds) {
+        void *params[] = {&dargs, &at};
+        const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kern),
+                                                        dim3(static_cast<unsigned>(r.size())), dim3(BLOCK), params,
+                                                        static_cast<unsigned>(lds), st);
+        if (e == hipErrorCooperativeLaunchTooLarge) {  // not all blocks fit at once on this device
+            (void)hipGetLastError();
+            FK_HIP(hipStreamSynchronize(st));
+            return false;
+        }
+        FK_HIP(e);
+        at += r.size();
+    }
+    FK_HIP(hipStreamSynchronize(st));  // args and table go out of scope
+    return true;
+}
+
+bool resident_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sys, double delta, int64_t max_iter, int chunk,
+                    std::vector<CgState> &state, std::vector<RuState> &ru) {
+    if (sys.empty()) return true;
+    const std::lock_guard<std::mutex> alone(resident_mutex(B.ctx->device));
+    B.started = false;
+    if (!launch_batch<512, 1, 1>(B, sys, delta, max_iter, chunk, 1) &&
+        !launch_batch<512, 2, 2>(B, sys, delta, max_iter, chunk, 1) &&
+        !launch_batch<512, 4, 4>(B, sys, delta, max_iter, chunk, kResBatchLaunches))
+        return false;
+    hipStream_t st = B.ctx->stream;
+    const size_t S = sys.size();
+    state.resize(S);
+    ru.resize(S);
+    FK_HIP(hipMemcpyAsync(state.data(), B.state.get(), S * sizeof(CgState), hipMemcpyDeviceToHost, st));
+    FK_HIP(hipMemcpyAsync(ru.data(), B.ru.get(), S * sizeof(RuState), hipMemcpyDeviceToHost, st));
+    FK_HIP(hipStreamSynchronize(st));
+    for (const RuState &r : ru)
+        if (r.status == FK_ERR_HIP) return false;  // a wait ran out (another process's launch)
     return true;
 }
 

@@ -218,3 +218,56 @@ def test_two_contexts_in_two_threads():
         dms[k].close()
         ctxs[k].close()
         assert len(got[k]) == 6 and all(np.array_equal(ref[k], u) for u in got[k])
+
+
+# (boxes nx, ny, nz, right-hand sides): one tiny mesh; rows 511, 512 and 513
+# wide of a block (7*73 = 511, 8*64, 9*57); one launch of 512, of 1024 rows a
+# block; several launches of 2048 with a mesh that ends a block exactly
+@pytest.mark.parametrize("boxes,nrhs", [
+    ([(1, 1, 1)], 1),
+    ([(6, 72, 1), (6, 6, 2), (7, 7, 7), (18, 8, 2), (1, 1, 400)], 4),
+    ([(20, 20, 20)] * 3 + [(3, 4, 5)], 2),
+    ([(32, 32, 20), (15, 15, 31), (30, 30, 30), (40, 40, 20)], 3),
+    ([(28, 28, 28)] * 7 + [(15, 15, 31), (2, 1, 3)], 3),
+])
+def test_batch(contexts, boxes, nrhs):
+    """Every system a group of blocks of its own; a system without a
+    right-hand side stays out. Potentials within the suite's 1e-9 of the
+    three-kernel batch at rtol 1e-12."""
+    from femeko_hip.batch import Batch
+
+    rng = np.random.default_rng(len(boxes) * 10 + nrhs)
+    meshes, mus, masks, gs = [], [], [], []
+    for b in boxes:
+        mesh = _box(*(max(v, 1) for v in b))
+        mask = np.zeros(mesh.nv, np.uint8)
+        mask[: (b[0] + 1) * 2] = 1
+        mask[-1] = 1
+        g = np.where(mask, rng.normal(size=(nrhs, mesh.nv)), 0.0)
+        meshes.append(mesh)
+        mus.append(MU0 * rng.uniform(1.0, 5.0, mesh.nt))
+        masks.append(mask)
+        gs.append(g)
+    if len(boxes) > 1:
+        gs[0][-1][:] = 0.0
+    out = []
+    for ctx in contexts:
+        b = Batch(meshes, nrhs=nrhs, ctx=ctx)
+        try:
+            b.set_coefficient(mus)
+            b.assemble()
+            b.set_dirichlet(masks, gs)
+            rep = b.solve(rtol=1e-12)
+            first = [b.potential(k) for k in range(b.nmesh)]
+            again = b.solve(rtol=1e-12)
+            assert all(np.array_equal(u, b.potential(k)) for k, u in enumerate(first))
+            assert np.array_equal(rep.iterations, again.iterations)
+            assert rep.relres.max() < 1e-12
+            with pytest.raises(FemekoHIPError):
+                b.solve(rtol=1e-12, max_iter=1)
+            out.append(first)
+        finally:
+            b.close()
+    for u, v in zip(*out):
+        for j in range(nrhs):
+            assert np.linalg.norm(u[j] - v[j]) <= 1e-9 * np.linalg.norm(v[j])
