@@ -161,8 +161,7 @@ void adjoint_field_target(fk_mesh *m, const uint8_t *target_host, const double *
     k_adjoint_grad<<<grid_for(nt, 256), 256, 0, st>>>(m->tet.get(), m->X.get(), m->Y.get(), m->Z.get(),
                                                       m->perm.get(), m->phi.get(), lam, nt, grad.get());
     FK_HIP(hipGetLastError());
-    FK_HIP(hipMemcpyAsync(grad_host, grad.get(), nt * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, grad_host, grad.get(), nt * sizeof(double));
     if (J_out) *J_out = J;
     if (iters_out) *iters_out = its;
 }

@@ -653,8 +653,7 @@ void local_stiffness(fk_mesh *m, const double *f, double *Ak_host) {
                                                             m->perm.get(), f ? coef.get() : nullptr, m->nt,
                                                             Ak.get());
     FK_HIP(hipGetLastError());
-    FK_HIP(hipMemcpyAsync(Ak_host, Ak.get(), 16 * m->nt * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, Ak_host, Ak.get(), 16 * m->nt * sizeof(double));
 }
 
 void tangential(fk_mesh *m, const double *H, const double *dmu, double *nzval_host) {
@@ -671,8 +670,7 @@ void tangential(fk_mesh *m, const double *H, const double *dmu, double *nzval_ho
                                                           val.get(), e0, e1);
     }
     FK_HIP(hipGetLastError());
-    FK_HIP(hipMemcpyAsync(nzval_host, val.get(), m->nnz * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, nzval_host, val.get(), m->nnz * sizeof(double));
     values_to_caller(m, nzval_host);
 }
 
@@ -688,8 +686,7 @@ void lagrange(fk_mesh *m, double *C_host) {
     }
     FK_HIP(hipGetLastError());
     NodesOut<double> out(m, C_host);
-    FK_HIP(hipMemcpyAsync(out.ptr, C.get(), m->nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, out.ptr, C.get(), m->nv * sizeof(double));
     out.commit();
 }
 
@@ -723,9 +720,7 @@ int fk_values(fk_mesh *m, double *values) {
     return guard(m->ctx, "fk_values", [&] {
         if (!m->have_values) fk::fail(FK_ERR_STATE, "matrix not assembled");
         fk::set_device(m->ctx);
-        FK_HIP(hipMemcpyAsync(values, m->val64.get(), m->nnz * sizeof(double), hipMemcpyDeviceToHost,
-                              m->ctx->stream));
-        FK_HIP(hipStreamSynchronize(m->ctx->stream));
+        fk::copy_out(m->ctx, values, m->val64.get(), m->nnz * sizeof(double));
         fk::values_to_caller(m, values);
     });
 }
@@ -736,9 +731,7 @@ int fk_values_f32(fk_mesh *m, float *values) {
         if (!m->have_values) fk::fail(FK_ERR_STATE, "matrix not assembled");
         fk::set_device(m->ctx);
         fk::make_val32(m);
-        FK_HIP(hipMemcpyAsync(values, m->val32.get(), m->nnz * sizeof(float), hipMemcpyDeviceToHost,
-                              m->ctx->stream));
-        FK_HIP(hipStreamSynchronize(m->ctx->stream));
+        fk::copy_out(m->ctx, values, m->val32.get(), m->nnz * sizeof(float));
         fk::values_to_caller(m, values);
     });
 }

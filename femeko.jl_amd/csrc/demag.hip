@@ -139,8 +139,7 @@ void demag_field(fk_mesh *m, const uint8_t *inside_host, const double *M_host, c
     k_div_volumes<<<grid_for(3 * nv, 256), 256, 0, st>>>(Hd.get(), vol.get(), nv);
     FK_HIP(hipGetLastError());
     NodesOut<double> Hd_out(m, Hd_host, 3);
-    FK_HIP(hipMemcpyAsync(Hd_out.ptr, Hd.get(), 3 * nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, Hd_out.ptr, Hd.get(), 3 * nv * sizeof(double));
     Hd_out.commit();
     if (iters_out) *iters_out = res.iters;
     if (relres_out) *relres_out = res.relres;

@@ -3,10 +3,15 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "femeko_hip.h"
@@ -159,13 +164,45 @@ struct TimingEvents {
 
 }  // namespace fk
 
+namespace fk {
+// Copies to pageable memory through a ring of pinned chunks that several
+// threads empty (transfer.hip); one copy at a time, made with the first one.
+struct HostLink {
+    explicit HostLink(int device);
+    ~HostLink();
+    void copy(void *to, const void *from, size_t bytes, hipStream_t st);  // returns when `to` holds the data
+
+  private:
+    void work(int t);
+    void share(int t);
+    hipError_t issue(size_t chunk);
+    int device;
+    HostBuf<char> ring;
+    std::vector<hipEvent_t> ev;
+    std::vector<std::thread> threads;
+    std::mutex use, mu;
+    std::condition_variable go, done;
+    uint64_t job = 0;
+    int left = 0;
+    bool quit = false;
+    char *dst = nullptr;
+    const char *src = nullptr;
+    size_t bytes = 0, piece = 0;
+    int takers = 1;
+    hipStream_t stream = nullptr;
+    hipError_t error = hipSuccess;
+};
+}  // namespace fk
+
 struct fk_context {
     int device = 0;
     hipStream_t stream = nullptr;
     int num_cus = 256;
     bool graphs = true;  // capture PCG iteration chunks in hipGraphs (FEMEKO_HIP_GRAPHS=0 disables)
+    bool one_shot = false;  // destroyed by the call that made it: no copy threads
     std::string err;
     fk::TimingEvents timing;
+    std::unique_ptr<fk::HostLink> link;
 };
 
 struct fk_mesh {
@@ -354,6 +391,8 @@ int solve_f32_free(fk_mesh *m, double *u, const double *b, double rtol, int64_t 
                    int64_t *iters, double *rr_out, double *bb_out);
 // one system of a batch: the stencil copy of its mesh (columns of n rows), its
 // potential and residual (a row's values us apart), scratch p of n values
+// device to caller memory on the context's stream; returns when it is there
+void copy_out(fk_context *ctx, void *to, const void *from, size_t bytes);
 struct ResidentSystem {
     const float *val32, *dinv;
     const double *val64, *diag64;

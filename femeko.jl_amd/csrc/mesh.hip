@@ -312,8 +312,7 @@ void element_volumes(fk_mesh *m, double *VE_host) {
     k_volumes<<<grid_for(m->nt, 256), 256, 0, st>>>(m->tet.get(), m->X.get(), m->Y.get(), m->Z.get(), m->nt,
                                                      m->perm.get(), d.get());
     FK_HIP(hipGetLastError());
-    FK_HIP(hipMemcpyAsync(VE_host, d.get(), m->nt * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, VE_host, d.get(), m->nt * sizeof(double));
 }
 
 }  // namespace fk
@@ -389,6 +388,7 @@ int fk_context_destroy(fk_context *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     for (hipEvent_t e : ctx->timing.ev) (void)hipEventDestroy(e);
+    ctx->link.reset();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return FK_OK;
@@ -495,15 +495,13 @@ int fk_pattern(fk_mesh *m, int32_t base, int32_t *rowptr, int32_t *colidx) {
     if (!m || !rowptr || !colidx || (base != 0 && base != 1)) return FK_ERR_INVALID_ARG;
     return guard(m->ctx, "fk_pattern", [&] {
         fk::set_device(m->ctx);
-        hipStream_t st = m->ctx->stream;
         if (m->reordered) {
             fk::build_caller_csr(m);
             std::copy(m->caller_rowptr.begin(), m->caller_rowptr.end(), rowptr);
             std::copy(m->caller_colidx.begin(), m->caller_colidx.end(), colidx);
         } else {
-            FK_HIP(hipMemcpyAsync(rowptr, m->rowptr.get(), (m->nv + 1) * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-            FK_HIP(hipMemcpyAsync(colidx, m->colidx.get(), m->nnz * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-            FK_HIP(hipStreamSynchronize(st));
+            fk::copy_out(m->ctx, rowptr, m->rowptr.get(), (m->nv + 1) * sizeof(int32_t));
+            fk::copy_out(m->ctx, colidx, m->colidx.get(), m->nnz * sizeof(int32_t));
         }
         if (base) {
             for (int64_t i = 0; i <= m->nv; ++i) rowptr[i] += 1;

@@ -167,8 +167,7 @@ void boundary_integral(fk_mesh *m, int64_t ns, const int32_t *sT_caller, const d
         k_boundary_integral<<<grid_for(ns, 256), 256, 0, st>>>(ns, dT.get(), dn.get(), dA.get(), F[0], F[1], F[2],
                                                                dids.get(), nids, base, rhs.get());
     FK_HIP(hipGetLastError());
-    FK_HIP(hipMemcpyAsync(rhs_out.ptr, rhs.get(), m->nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, rhs_out.ptr, rhs.get(), m->nv * sizeof(double));
     rhs_out.commit();
 }
 
@@ -272,8 +271,7 @@ void solve_neumann(fk_mesh *m, const double *b_host, double rtol, int64_t max_it
     NodesOut<double> u_out(m, u_host);
     FK_HIP(hipMemcpyAsync(m->w64.r.get(), b_in.ptr, m->nv * sizeof(double), hipMemcpyHostToDevice, st));
     const NeumannResult res = solve_neumann_dev(m, rtol, max_iter, nullptr);
-    FK_HIP(hipMemcpyAsync(u_out.ptr, m->w64.x.get(), m->nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, u_out.ptr, m->w64.x.get(), m->nv * sizeof(double));
     u_out.commit();
     if (mult_out) *mult_out = res.multiplier;
     if (iters_out) *iters_out = res.iters;
@@ -300,6 +298,7 @@ static void scalar_potential(double *u, const double *p, const int32_t *t, const
     } mesh;
     int s = fk_context_create(0, &ctx.c);
     if (s != FK_OK) fail(s, "no GPU context on device 0");
+    ctx.c->one_shot = true;
     s = fk_mesh_create(ctx.c, p, nv, t, nt, 0, VE, &mesh.m);
     if (s != FK_OK) fail(s, std::string("mesh: ") + fk_context_last_error(ctx.c));
     fk_mesh *m = mesh.m;
@@ -344,8 +343,7 @@ static void scalar_potential(double *u, const double *p, const int32_t *t, const
     k_shift<<<grid_for(nv, 256), 256, 0, st>>>(m->w64.x.get(), dd > 0.0 ? du / dd : 0.0, nv);
     FK_HIP(hipGetLastError());
     NodesOut<double> u_out(m, u);
-    FK_HIP(hipMemcpyAsync(u_out.ptr, m->w64.x.get(), nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, u_out.ptr, m->w64.x.get(), nv * sizeof(double));
     u_out.commit();
 }
 

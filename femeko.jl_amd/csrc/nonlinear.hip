@@ -506,8 +506,7 @@ double line_search(fk_mesh *m, double *u_host, const double *du_host, const doub
     const double residue = line_search_dev(m, u.get(), du.get(), rhs.get(), min_step, y.get(), nullptr, &moved);
     if (moved) {
         NodesOut<double> uo(m, u_host);
-        FK_HIP(hipMemcpyAsync(uo.ptr, u.get(), nv * sizeof(double), hipMemcpyDeviceToHost, st));
-        FK_HIP(hipStreamSynchronize(st));
+        copy_out(m->ctx, uo.ptr, u.get(), nv * sizeof(double));
         uo.commit();
     }
     return residue;
@@ -639,8 +638,7 @@ void get_coefficient(fk_mesh *m, double *f_host) {
     DevBuf<double> out(m->nt);
     k_scatter_coef<<<grid_for(m->nt, 256), 256, 0, st>>>(m->coef.get(), m->perm.get(), m->nt, out.get());
     FK_HIP(hipGetLastError());
-    FK_HIP(hipMemcpyAsync(f_host, out.get(), m->nt * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, f_host, out.get(), m->nt * sizeof(double));
 }
 
 }  // namespace fk

@@ -2264,8 +2264,7 @@ void solve_rhs(fk_mesh *m, const double *b, double rtol, int64_t max_iter, doubl
     NodesOut<double> x_out(m, x);
     FK_HIP(hipMemcpyAsync(w.r.get(), b_in.ptr, m->nv * sizeof(double), hipMemcpyHostToDevice, st));
     const CgState s = run_pcg<double>(m, rtol, max_iter, -1.0);
-    FK_HIP(hipMemcpyAsync(x_out.ptr, w.x.get(), m->nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    FK_HIP(hipStreamSynchronize(st));
+    copy_out(m->ctx, x_out.ptr, w.x.get(), m->nv * sizeof(double));
     x_out.commit();
     if (iters) *iters = s.iters;
     if (relres) *relres = s.bb > 0 ? std::sqrt(s.rr / s.bb) : 0.0;
@@ -2286,8 +2285,8 @@ void field(fk_mesh *m, double *H, double *Hn, double *energy) {
                                    energy ? coef_caller_order(m, true) : nullptr, m->nt, H ? dH.get() : nullptr,
                                    Hn ? dHn.get() : nullptr, m->part_misc.get());
     FK_HIP(hipGetLastError());
-    if (H) FK_HIP(hipMemcpyAsync(H, dH.get(), 3 * m->nt * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (Hn) FK_HIP(hipMemcpyAsync(Hn, dHn.get(), m->nt * sizeof(double), hipMemcpyDeviceToHost, st));
+    if (H) copy_out(m->ctx, H, dH.get(), 3 * m->nt * sizeof(double));
+    if (Hn) copy_out(m->ctx, Hn, dHn.get(), m->nt * sizeof(double));
     FK_HIP(hipMemcpyAsync(m->hpart.ptr, m->part_misc.get(), nb * sizeof(double), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
     if (energy) {
@@ -2383,8 +2382,7 @@ int fk_potential(fk_mesh *m, double *phi) {
         if (!m->have_phi) fk::fail(FK_ERR_STATE, "no potential");
         fk::set_device(m->ctx);
         fk::NodesOut<double> out(m, phi);
-        FK_HIP(hipMemcpyAsync(out.ptr, m->phi.get(), m->nv * sizeof(double), hipMemcpyDeviceToHost, m->ctx->stream));
-        FK_HIP(hipStreamSynchronize(m->ctx->stream));
+        fk::copy_out(m->ctx, out.ptr, m->phi.get(), m->nv * sizeof(double));
         out.commit();
     });
 }
