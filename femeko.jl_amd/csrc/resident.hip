@@ -24,6 +24,14 @@
 // lies in LDS; each window element outside the own rows belongs to one thread,
 // which keeps its z in a register. 2 R + 4 m of them are exchanged per
 // iteration for the 15-point patterns of an m^3 grid.
+//
+// Larger meshes go by bricks: with P the offset of the next plane, a block owns
+// the rows z P + t of a few planes z and a run of t. Its halo, a plane above
+// and below and a reach of a + 1 rows at both ends of every run, is far smaller
+// than the windows (n = 160: 7.3k rows beside 16.8k own ones, where windows
+// take 33k and do not fit), and a row's backward values are the forward ones
+// the block has just read for the plane below, from L2. p lies in LDS alone, and
+// only rows within reach of the brick's faces send their w.
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -63,6 +71,9 @@ struct ResidentArgs {
     const uint16_t *sidx;
     const int32_t *halo_ptr, *halo;
     int32_t nslices, spare;       // LDS index of the spare element
+    // bricks: rows z P + t, 0 <= t < P; a block owns len rows of several planes
+    int32_t P, len, reach, S;     // reach of the stencil in t; S = len + 2 reach, a plane in LDS
+    int32_t groups;               // blocks side by side in a plane
     double bb_ref, rtol;
     int64_t max_iter;
     // residual replacement (FP32 recursion, FP64 solution u)
@@ -99,9 +110,25 @@ __device__ __forceinline__ int32_t window_row(Args &A, int32_t i0, int32_t li) {
     return li < A.wbeg[kResWindows] ? i0 + li + d : -1;
 }
 
+// a row that no buffer holds: loads of it read zero, stores are dropped
+constexpr int32_t kNoRow = 0x10000000;
+
+// rows per thread whose x waits in LDS, past the windows: all of the FP64
+// shapes with many rows, and half of the FP32 bricks that would spill
 template <typename T>
-constexpr bool x_in_lds(int rpt) {
-    return sizeof(T) == 8 && rpt >= 4;
+constexpr int x_in_lds(int rpt, bool brick) {
+    return sizeof(T) == 8 ? (rpt < 4 ? 0 : rpt > 16 ? 9 : rpt > 14 ? 12 : rpt) : brick && rpt > 22 ? rpt * 3 / 5 : 0;
+}
+
+// 1 / v to the last bit or so; v = 0: 0
+__device__ __forceinline__ float reciprocal(float v) {
+    const float y = __builtin_amdgcn_rcpf(v);
+    return v != 0.f ? fmaf(y, fmaf(-v, y, 1.f), y) : 0.f;
+}
+__device__ __forceinline__ double reciprocal(double v) {
+    double y = __builtin_amdgcn_rcp(v);
+    y = fma(y, fma(-v, y, 1.0), y);
+    return v != 0.0 ? fma(y, fma(-v, y, 1.0), y) : 0.0;
 }
 
 constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursion gives up
@@ -113,6 +140,10 @@ constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursio
 // NE > 0: the SELL copy instead of the stencil, rows of at most NE entries.
 // The own rows lie first in LDS, the rows of the block's halo list after them,
 // and every entry keeps its value and the LDS index of its column.
+//
+// NE < 0: a brick of the stencil copy, runs of up to -NE x BLOCK rows in each of
+// its planes, NK rows' values in flight. Slots past a run's end hold no row:
+// their d, z and w are 0.
 //
 // REFINE (T = float): the reliable updates of solve.hip inside the launch. At
 // the end of every G iterations in which ||r||^2 has fallen by delta2 since
@@ -127,17 +158,32 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
     T *win = reinterpret_cast<T *>(lds_raw);
     __shared__ double sh[kReduceShared];
     constexpr int K = kResK, R = BLOCK * RPT;
-    constexpr bool GEN = NE > 0;
+    constexpr bool GEN = NE > 0, BRICK = NE < 0;
+    constexpr int TP = BRICK ? -NE : 1, BZ = RPT / TP;  // runs of BLOCK rows in a plane of a brick, planes
+    static_assert(!BRICK || (NK > 0 && RPT % NK == 0 && RPT % TP == 0), "whole planes and turns of the ring");
     constexpr int E = GEN ? NE : 2 * K;  // entries per row: K forward, then K backward ones
     static_assert(!GEN || NK == RPT, "SELL values are not streamed");
-    // x of the FP64 shapes with many rows per thread waits in LDS, past the windows
-    constexpr bool XLDS = x_in_lds<T>(RPT);
-    T *xs = win + (GEN ? A.spare : A.wbeg[kResWindows]) + 1;
+    constexpr int XL = x_in_lds<T>(RPT, BRICK);
+    T *xs = win + (GEN || BRICK ? A.spare : A.wbeg[kResWindows]) + 1;
     constexpr bool AHEAD = RPT > 1 && (sizeof(T) == 4 || (!GEN && RPT <= 3));
     const int32_t tid = threadIdx.x;
     const AgentRows<T> rows(A.w, A.stride);
     const ValueColumns<T> vals(A.val, A.K, A.ld);
     const int32_t n = A.n, lown = GEN ? 0 : A.lown;
+    const int32_t bt = BRICK ? (i0 % A.P) : 0, blen = BRICK ? min(A.len, A.P - bt) : 0;
+    const int32_t hbase = BRICK ? i0 - A.P - A.reach : 0;  // row of LDS element 0
+    // row of thread t's j-th own element, n or more if there is none, and its LDS index
+    const auto own_row = [&](int j, int32_t t) {
+        if constexpr (BRICK) {
+            const int32_t in = (j % TP) * BLOCK + t, first = i0 + (j / TP) * A.P;
+            return in < min(blen, n - first) ? first + in : kNoRow;
+        } else {
+            return i0 + j * BLOCK + t;
+        }
+    };
+    const auto own_lds = [&](int j, int32_t t) {
+        return BRICK ? lown + (j / TP) * A.S + (j % TP) * BLOCK + t : lown + j * BLOCK + t;
+    };
     const int32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int32_t h0 = GEN ? A.halo_ptr[i0 / R] : 0, nh = GEN ? A.halo_ptr[i0 / R + 1] - h0 : 0;
     uint32_t tag = 1;
@@ -147,7 +193,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
     for (int j = 0; j < RPT; ++j) {
-        const int32_t row = i0 + j * BLOCK + tid;
+        const int32_t row = own_row(j, tid);
         if (row >= n) continue;
         const T dj = A.dinv[row];
         T r = T(0);
@@ -165,16 +211,23 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
     while (code < 0) {
         // ---- a run of iterations from z (exchanged) and p: state into registers
         const int32_t tl = fresh(tid);
-        T d[RPT], g[RPT], x[XLDS ? 1 : RPT], z[RPT], p[RPT], w[RPT];
+        T d[RPT], g[BRICK ? 1 : RPT], x[XL < RPT ? RPT - XL : 1], z[RPT], p[BRICK ? 1 : RPT], w[RPT];
         T zw[U];
-        T v[NK > 0 ? NK : 1][E];
+        [[maybe_unused]] T v[NK > 0 ? NK : 1][E];
         [[maybe_unused]] uint32_t pk[GEN ? RPT : 1][GEN ? NE / 2 : 1];  // LDS indices of two entries
-        [[maybe_unused]] int32_t hrow[GEN ? U : 1];                     // rows of this thread's halo elements
+        // rows of this thread's halo elements; bricks: LDS index and, from bit
+        // 16, plane slot of each, the sign bit where there is no row
+        [[maybe_unused]] int32_t hrow[GEN || BRICK ? U : 1];
+        const auto xj = [&](int j, int32_t t) -> T & { return j < XL ? xs[j * BLOCK + t] : x[j < XL ? 0 : j - XL]; };
         // LDS index and row of the u-th window element (spare: none)
         const auto element = [&](int u, int32_t t, int32_t &row) {
             if constexpr (GEN) {
                 row = hrow[u];
                 return row >= 0 ? R + t + u * BLOCK : A.spare;
+            } else if constexpr (BRICK) {
+                const int32_t h = fresh(hrow[u]), li = h & 0xffff;
+                row = h < 0 ? kNoRow : hbase + li + (h >> 16) * (A.P - A.S);
+                return li;
             } else {
                 const int32_t li = window_lds(A, R, t + u * BLOCK);
                 row = window_row(A, i0, li);
@@ -186,7 +239,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
 #pragma unroll
             for (int k = 0; k < K; ++k) {
                 o[k] = o[K + k] = T(0);
-                if (k < A.K) {
+                if (BRICK || k < A.K) {
                     o[k] = vals.load(k, row);
                     o[K + k] = vals.load(k, row - A.off[k]);
                 }
@@ -194,19 +247,21 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
         };
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
-            const int32_t row = i0 + j * BLOCK + tl, at = min(row, n - 1);
-            const T dj = A.dinv[at], pj = restart ? T(0) : A.p[at];
+            const int32_t row = own_row(j, tl), at = min(row, n - 1);
+            const T dj = A.dinv[at], pj = restart || BRICK ? T(0) : A.p[at];
             z[j] = rows.load(tag, row);  // 0 past the last row
             d[j] = row < n ? dj : T(0);
-            p[j] = restart || row >= n ? z[j] : pj;
-            if (XLDS)
-                xs[j * BLOCK + tl] = T(0);
-            else
-                (XLDS ? xs[j * BLOCK + tl] : x[XLDS ? 0 : j]) = T(0);
-            if (restart) win[lown + j * BLOCK + tl] = p[j];
+            if constexpr (!BRICK) p[j] = restart || row >= n ? z[j] : pj;
+            xj(j, tl) = T(0);
+            // a brick's p stays in LDS; its elements past a run belong to the halo
+            if (restart && (!BRICK || (j % TP) * BLOCK + tl < blen))
+                win[own_lds(j, tl)] = BRICK ? z[j] : p[BRICK ? 0 : j];
+            if (BRICK && j % TP == TP - 1) __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (!BRICK) {
 #pragma unroll
-        for (int j = 0; j < RPT; ++j) g[j] = d[j] != T(0) ? T(1) / d[j] : T(0);
+            for (int j = 0; j < RPT; ++j) g[j] = d[j] != T(0) ? T(1) / d[j] : T(0);
+        }
         if constexpr (GEN) {
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
@@ -233,6 +288,18 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                 const int32_t e = tl + u * BLOCK;
                 hrow[u] = e < nh ? A.halo[h0 + e] : -1;
             }
+        } else if constexpr (BRICK) {
+            // the planes below and above in full, then both ends of the own planes
+            const int32_t w2 = 2 * A.reach, many = 2 * A.S + BZ * w2;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int32_t e = tl + u * BLOCK, f = e - 2 * A.S, q = f < 0 ? 0 : f / w2, r = f - q * w2;
+                const int32_t slot = f >= 0 ? 1 + q : e < A.S ? 0 : BZ + 1;
+                const int32_t in = f >= 0 ? (r < A.reach ? r : blen + r) : e < A.S ? e : e - A.S;
+                const int32_t row = hbase + slot * A.P + in;
+                const bool have = e < many && row >= 0 && row < n;
+                hrow[u] = (e < many ? slot * A.S + in : A.spare) | (have ? slot << 16 : INT32_MIN);
+            }
         } else {
 #pragma unroll
             for (int j = 0; j < NK; ++j) load_row(i0 + j * BLOCK + tl, v[j]);
@@ -245,6 +312,11 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             if (restart) win[li] = zw[u];
         }
         __syncthreads();
+        // a brick's values: NK rows in flight, also over the end of an iteration
+        if constexpr (BRICK) {
+#pragma unroll
+            for (int j = 0; j < NK; ++j) load_row(own_row(j, tl), v[j]);
+        }
         [[maybe_unused]] bool moved = false;  // an iteration done in this run
         [[maybe_unused]] int act = 0;         // why it ended: 1 replace r, 2 drop x and restart
         while (true) {
@@ -252,6 +324,40 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             // q = A p in difference form; w = D^-1 q
 #pragma unroll
             for (int k = 0; k < 5; ++k) s[k] = 0.0;
+            if constexpr (BRICK) {
+#pragma unroll
+                for (int j = 0; j < RPT; ++j) {
+                    const int32_t t = fresh(tid), in = (j % TP) * BLOCK + t, row = own_row(j, t);
+                    // the seven offsets are 1, a, a + 1, P, P + 1, P + a, P + a + 1:
+                    // adjacent neighbours come with one LDS instruction
+                    const T *c = win + own_lds(j, t);
+                    const int32_t a = A.lf[1] - lown, sa = A.S + a;
+                    const T *fa = c + a, *ba = c - a, *fs = c + A.S, *bs = c - A.S, *fsa = c + sa, *bsa = c - sa;
+                    const T nb[E] = {c[1],  fa[0], fa[1],  fs[0], fs[1],  fsa[0], fsa[1],
+                                     c[-1], ba[0], ba[-1], bs[0], bs[-1], bsa[0], bsa[-1]};
+                    const T pj = c[0];
+                    T a0 = T(0), a1 = T(0);
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        a0 += v[j % NK][k] * (nb[k] - pj);
+                        a1 += v[j % NK][K + k] * (nb[K + k] - pj);
+                    }
+                    const T q = d[j] != T(0) ? a0 + a1 : T(0);
+                    w[j] = d[j] * q;
+                    // only the rows that other blocks reach go out
+                    const bool inner = j >= TP && j < RPT - TP && in >= A.reach && in < blen - A.reach;
+                    rows.store(tag, inner ? kNoRow : row, w[j]);
+                    load_row(own_row((j + NK) % RPT, t), v[j % NK]);
+                    const double zd = static_cast<double>(z[j]), qd = static_cast<double>(q);
+                    const double rd = static_cast<double>(reciprocal(d[j]) * z[j]);
+                    s[0] += static_cast<double>(d[j] != T(0) ? pj : T(0)) * qd;  // past a run: any LDS word
+                    s[1] += rd * zd;
+                    s[2] += qd * zd;
+                    s[3] += qd * static_cast<double>(w[j]);
+                    s[4] += rd * rd;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
             [[maybe_unused]] T sv[E];  // values of the streamed row at hand
             if constexpr (NK < RPT) load_row(i0 + NK * BLOCK + fresh(tid), sv);
             // the neighbours of a row are loaded together, and where registers
@@ -307,6 +413,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                 s[4] += rd * rd;
                 __builtin_amdgcn_sched_barrier(0);
             }
+            }
             alive = all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
             T ww[U];
             const int32_t ft = fresh(tid);
@@ -351,10 +458,21 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             ++it;
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
-                (XLDS ? xs[j * BLOCK + ft] : x[XLDS ? 0 : j]) += alpha * p[j];
-                z[j] -= alpha * w[j];
-                p[j] = z[j] + beta * p[j];
-                win[lown + j * BLOCK + ft] = p[j];
+                if constexpr (BRICK) {
+                    if ((j % TP) * BLOCK + ft < blen) {
+                        T &pj = win[own_lds(j, ft)];
+                        const T old = pj;
+                        xj(j, ft) += alpha * old;
+                        z[j] -= alpha * w[j];
+                        pj = z[j] + beta * old;
+                    }
+                    if (j % TP == TP - 1) __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    xj(j, ft) += alpha * p[j];
+                    z[j] -= alpha * w[j];
+                    p[j] = z[j] + beta * p[j];
+                    win[lown + j * BLOCK + ft] = p[j];
+                }
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -368,7 +486,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
         if constexpr (!REFINE) {
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
-                const int32_t row = i0 + j * BLOCK + tid;
+                const int32_t row = own_row(j, tid);
                 // One Jacobi step of 1/3 on the way out. The largest eigenvalues
                 // of D^-1 A are those of slivers, 2 to 4 (4: flat, four nodes; the
                 // scaled matrix of an element with parallel gradients has rank one
@@ -377,11 +495,10 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                 // sliver does. The step takes two thirds or more off them and
                 // lengthens no other mode: largest error of H over 24 jittered
                 // meshes of 63^3 cells 1.6e-7 of its rms without, 6.6e-9 to 3e-8 with.
-                const T xj = XLDS ? xs[j * BLOCK + tid] : x[XLDS ? 0 : j];
-                if (row < n) A.x[row] = code == FK_OK ? xj + T(1.0 / 3.0) * z[j] : xj;
+                const T xr = xj(j, tid);
+                if (row < n) A.x[row] = code == FK_OK ? xr + T(1.0 / 3.0) * z[j] : xr;
             }
         } else {
-            static_assert(!XLDS, "the replacement folds x from registers");
             // ---- replacement: nothing but x and p leaves the registers
             if (act == 3) {
                 code = FK_ERR_HIP;
@@ -395,10 +512,10 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                 const double inv_s = 1.0 / A.s;
 #pragma unroll
                 for (int j = 0; j < RPT; ++j) {
-                    const int32_t row = i0 + j * BLOCK + tc;
+                    const int32_t row = own_row(j, tc);
                     if (row < n) {
-                        sol.store(0, row * A.us, A.u[at(row)] + inv_s * static_cast<double>(x[XLDS ? 0 : j]));
-                        A.p[row] = p[j];
+                        sol.store(0, row * A.us, A.u[at(row)] + inv_s * static_cast<double>(xj(j, tc)));
+                        if constexpr (!BRICK) A.p[row] = p[j];
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -420,7 +537,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             s[0] = 0.0;
 #pragma unroll 1
             for (int j = 0; j < RPT; ++j) {
-                const int32_t row = i0 + j * BLOCK + tc;
+                const int32_t row = own_row(j, tc);
                 if (row >= n) continue;
                 const T dj = A.dinv[row];
                 double v = dj != T(0) ? A.r64[at(row)] : 0.0;
@@ -493,8 +610,15 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
 
 template <typename T, int BLOCK, int RPT, int NK, int U, bool REFINE, int NE>
 __global__ __launch_bounds__(BLOCK) void k_resident_pcg(const ResidentArgs<T> A) {
-    resident_solve<T, BLOCK, RPT, NK, U, REFINE, NE>(A, static_cast<int>(blockIdx.x),
-                                                     logical_block(A.nb) * (BLOCK * RPT));
+    const int32_t lb = logical_block(A.nb);
+    if constexpr (NE < 0) {
+        // a block past the last plane owns nothing
+        const int32_t z0 = lb / A.groups * (RPT / -NE), t0 = lb % A.groups * A.len;
+        const int32_t last = (A.n - 1) / A.P + 1;
+        resident_solve<T, BLOCK, RPT, NK, U, REFINE, NE>(A, static_cast<int>(blockIdx.x), min(z0, last) * A.P + t0);
+    } else {
+        resident_solve<T, BLOCK, RPT, NK, U, REFINE, NE>(A, static_cast<int>(blockIdx.x), lb * (BLOCK * RPT));
+    }
 }
 
 // Several systems in one launch: block b is block first[b].y of system
@@ -569,15 +693,66 @@ static bool place_windows(const int32_t *off, int K, int R, ResidentArgs<T> &A, 
     return true;
 }
 
+// The bricks of BZ planes whose runs fill TP x BLOCK threads, at most `most` of
+// them, for the offsets 1, a, a + 1, P, P + 1, P + a, P + a + 1 of a grid of
+// boxes cut along their diagonals. Nothing else is asked of the numbering: a
+// row is z P + t by definition, and t may run past a plane's end into the next.
+template <typename T>
+static bool place_bricks(const int32_t *off, int K, int64_t n, int most, int BZ, int run, ResidentArgs<T> &A, int *nb,
+                         int32_t *elements, int32_t *halo) {
+    if (K != 7) return false;
+    const int64_t a = off[1], P = off[3], reach = a + 1;
+    if (off[0] != 1 || off[2] != a + 1 || off[4] != P + 1 || off[5] != P + a || off[6] != P + a + 1) return false;
+    const int64_t planes = (n + P - 1) / P, layers = (planes + BZ - 1) / BZ;
+    if (layers > most) return false;
+    const int64_t groups = most / layers, len = (P + groups - 1) / groups;
+    const int64_t S = len + 2 * reach, total = (BZ + 2) * S + run - len;
+    if (len > run || 2 * reach >= P || total > 0xffff) return false;
+    A.P = static_cast<int32_t>(P);
+    A.len = static_cast<int32_t>(len);
+    A.reach = static_cast<int32_t>(reach);
+    A.S = static_cast<int32_t>(S);
+    A.groups = static_cast<int32_t>((P + len - 1) / len);
+    A.lown = static_cast<int32_t>(S + reach);
+    for (int k = 0; k < kResK; ++k) {
+        const int64_t o = k < 3 ? off[k] : off[k] - P + S;
+        A.off[k] = off[k];
+        A.lf[k] = static_cast<int32_t>(A.lown + o);
+        A.lb[k] = static_cast<int32_t>(A.lown - o);
+    }
+    A.spare = *elements = static_cast<int32_t>(total);
+    *halo = static_cast<int32_t>(2 * S + 2 * reach * BZ);
+    *nb = static_cast<int>(layers * A.groups);
+    // neighbouring bricks on one XCD: n = 160 FP32 32.9 -> 31.7 us an iteration, n = 100 FP64 14.6 -> 13.7
+    if (*nb > kNumXcd) *nb = std::min((*nb + kNumXcd - 1) / kNumXcd * kNumXcd, most);
+    return true;
+}
+
+// halo elements per thread of a brick at most: its two outer planes, and the
+// ends of the inner ones up to a reach of 170 (FP64: 128)
+template <typename T>
+constexpr int brick_halo(int BZ, int TP) {
+    return 2 * TP + (sizeof(T) == 4 ? (2 * BZ + 6) / 3 : (BZ + 3) / 2);
+}
+
 template <typename T, int BLOCK, int RPT, int NK, bool REFINE = false, int NE = 0>
 static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
-    constexpr int R = BLOCK * RPT, U = NE > 0 ? (RPT <= 2 ? 4 * RPT : 3 * RPT) : 2 * RPT + 2;
+    constexpr int R = BLOCK * RPT;
+    constexpr int U = NE > 0   ? (RPT <= 2 ? 4 * RPT : 3 * RPT)
+                      : NE < 0 ? brick_halo<T>(NE < 0 ? RPT / -NE : 1, -NE)
+                               : 2 * RPT + 2;
     const int most = std::min(m->ctx->num_cus, kMaxResidentBlocks);
     int nb = static_cast<int>((m->nv + R - 1) / R);
     if (nb > most) return false;
-    // streamed values: one band of rows per XCD
-    if (NK < RPT && nb > kNumXcd) nb = std::min((nb + kNumXcd - 1) / kNumXcd * kNumXcd, most);
     int32_t elements = 0;
+    if constexpr (NE < 0) {
+        int32_t halo = 0;
+        if (!place_bricks<T>(m->st_off, m->st_K, m->nv, most, RPT / -NE, BLOCK * -NE, A, &nb, &elements, &halo) ||
+            halo > U * BLOCK)
+            return false;
+    }
+    // streamed values: one band of rows per XCD
+    if (NE == 0 && NK < RPT && nb > kNumXcd) nb = std::min((nb + kNumXcd - 1) / kNumXcd * kNumXcd, most);
     if constexpr (NE > 0) {
         if (m->res_R != R || m->res_halo_max > U * BLOCK) return false;
         elements = R + m->res_halo_max;
@@ -588,14 +763,14 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
         A.halo_ptr = m->res_halo_ptr.get();
         A.halo = m->res_halo.get();
         A.nslices = static_cast<int32_t>(m->nslices);
-    } else {
+    } else if constexpr (NE == 0) {
         if (!place_windows<T>(m->st_off, m->st_K, R, A, &elements) || elements - R > U * BLOCK) return false;
     }
-    const size_t lds = (static_cast<size_t>(elements) + 1 + (x_in_lds<T>(RPT) ? R : 0)) * sizeof(T);
+    const size_t lds = (static_cast<size_t>(elements) + 1 + x_in_lds<T>(RPT, NE < 0) * BLOCK) * sizeof(T);
     if (lds > static_cast<size_t>(kResLdsMax)) return false;
     A.nb = nb;
     // rows past the last, as far as the last block's windows reach, read zero
-    const int64_t reach = static_cast<int64_t>(nb) * R + (NE > 0 ? 0 : m->st_off[m->st_K - 1] + R);
+    const int64_t reach = NE < 0 ? m->nv : static_cast<int64_t>(nb) * R + (NE > 0 ? 0 : m->st_off[m->st_K - 1] + R);
     const int64_t stride = (reach + 63) / 64 * 64;
     hipStream_t st = m->ctx->stream;
     m->res_slots.ensure(reduce_words(kMaxResidentBlocks));
@@ -629,6 +804,43 @@ static int64_t rows_per_block(const fk_mesh *m) {
     return (m->nv + most - 1) / most;
 }
 
+// Bricks of BZ planes and runs of up to TP x 512 rows in a plane, the values
+// streamed one row ahead: the first shape of the list, by slots per thread,
+// whose threads, halo registers and LDS cover the mesh with one brick per CU.
+// The shapes are those that leave few slots empty on some mesh: an m^3 grid
+// wastes 1 to 20% of them. Measured per iteration (us; windows or, from the
+// second dash on, the three kernels in brackets), Kuhn meshes of n cells per side:
+//   FP64  n = 80  8.8 (10.9)   n = 90 11.6 (14.1)   n = 95 11.7 (18.5)   n = 100 13.7 (22.2)
+//         n = 105 16 (41.5)    n = 118 21 (52.7)    n = 125 24 (60.0)    n = 130 35 (67.5)
+//   FP32  n = 80  7.7 (8.7)    n = 95 9.3 (11.5)    n = 100 11.0 (13.5)  n = 115 14.3 (20.5)
+//         n = 126 17 (28.8)    n = 140 23.6 (45.6)  n = 150 27 (53.8)    n = 160 31.7 (61.8)
+// More rows in flight (2 or 3 per thread) were no faster at any size: n = 160
+// 40.0 us with 3, where they spill, n = 115 14.9 with 2 or 3. What bounds the
+// larger ones is the value stream from the MALL (7 columns, 117 MB at n = 160
+// in about 25 of the 31.7 us), then the exchange and the all-reduce (6 to 8).
+//
+// Up to four rows per thread the windows, which keep the values in registers,
+// are faster: FP64 n = 76 7.1 us against 7.8, n = 70 6.3 against 7.9.
+constexpr int64_t kBrickRows = 2048;
+
+template <typename T, int BZ, int TP>
+static bool brick(fk_mesh *m, ResidentArgs<T> &A) {
+    return launch_resident<T, 512, BZ * TP, 1, sizeof(T) == 4, -TP>(m, A);
+}
+static bool launch_bricks(fk_mesh *m, ResidentArgs<double> &A) {
+    return brick<double, 5, 1>(m, A) || brick<double, 6, 1>(m, A) || brick<double, 7, 1>(m, A) ||
+           brick<double, 8, 1>(m, A) || brick<double, 9, 1>(m, A) || brick<double, 5, 2>(m, A) ||
+           brick<double, 11, 1>(m, A) || brick<double, 6, 2>(m, A) || brick<double, 7, 2>(m, A) ||
+           brick<double, 8, 2>(m, A) || brick<double, 9, 2>(m, A);
+}
+static bool launch_bricks(fk_mesh *m, ResidentArgs<float> &A) {
+    return brick<float, 5, 1>(m, A) || brick<float, 6, 1>(m, A) || brick<float, 7, 1>(m, A) ||
+           brick<float, 9, 1>(m, A) || brick<float, 5, 2>(m, A) || brick<float, 6, 2>(m, A) ||
+           brick<float, 7, 2>(m, A) || brick<float, 8, 2>(m, A) || brick<float, 9, 2>(m, A) ||
+           brick<float, 7, 3>(m, A) || brick<float, 8, 3>(m, A) || brick<float, 9, 3>(m, A) ||
+           brick<float, 10, 3>(m, A) || brick<float, 11, 3>(m, A) || brick<float, 12, 3>(m, A);
+}
+
 // Rows per block by the number of rows: the smallest shape of the list with
 // which at most one block per CU covers them. Few rows per thread leave room
 // for all their matrix values in registers (NK = RPT) and shorten every step
@@ -644,6 +856,7 @@ static int64_t rows_per_block(const fk_mesh *m) {
 // iteration: the windows of more rows per block exceed the LDS.
 static bool launch_by_rows(fk_mesh *m, ResidentArgs<double> &A) {
     const int64_t per = rows_per_block(m);
+    if (per > kBrickRows && launch_bricks(m, A)) return true;
     if (per <= 512) return launch_resident<double, 512, 1, 1>(m, A);
     if (per <= 1024) return launch_resident<double, 512, 2, 2>(m, A);
     if (per <= 1536) return launch_resident<double, 512, 3, 3>(m, A);
@@ -663,6 +876,7 @@ static bool launch_by_rows(fk_mesh *m, ResidentArgs<double> &A) {
 //   n = 115 512 x 12 20   (31)       n = 126 512 x 16 28.1 (35.6)
 static bool launch_by_rows(fk_mesh *m, ResidentArgs<float> &A) {
     const int64_t per = rows_per_block(m);
+    if (per > kBrickRows && launch_bricks(m, A)) return true;
     if (per <= 512) return launch_resident<float, 512, 1, 1, true>(m, A);
     if (per <= 1024) return launch_resident<float, 512, 2, 2, true>(m, A);
     if (per <= 1536) return launch_resident<float, 512, 3, 3, true>(m, A);

@@ -105,8 +105,30 @@ def test_launch_shapes_f32(contexts, n):
     _both(contexts, pr.mesh, pr.mu, pr.mask, pr.g, precision="f32", fmt="stencil")
 
 
+# bricks: the last n of a shape and the first of the next, up to the last mesh
+# that fits (FP64 n = 131, FP32 n = 162) and one past it (three kernels)
+@pytest.mark.parametrize("precision,n", [("f64", n) for n in (83, 84, 95, 102, 103, 107, 113, 119, 127, 130)]
+                         + [("f32", n) for n in (83, 87, 102, 118, 130, 134, 143, 151, 162, 163)])
+def test_brick_shapes(contexts, precision, n):
+    pr = W.linear(n)
+    _both(contexts, pr.mesh, pr.mu, pr.mask, pr.g, precision=precision, fmt="stencil")
+
+
+# bricks of grids that are no cubes: two runs per plane over 120 layers; one
+# layer of few planes; short last runs and last layers
+@pytest.mark.parametrize("dims", [(30, 30, 600), (400, 400, 3), (230, 47, 55), (61, 201, 43), (90, 13, 500)])
 @pytest.mark.parametrize("precision", ["f64", "f32"])
-@pytest.mark.parametrize("n", [12, 34])
+def test_brick_grids(contexts, dims, precision):
+    mesh = _box(*dims)
+    rng = np.random.default_rng(5)
+    mu = MU0 * rng.uniform(1.0, 50.0, mesh.nt)
+    mask = ((mesh.p == 0.0) | (mesh.p == np.array(dims, float)[:, None])).any(axis=0)
+    g = np.where(mask, rng.normal(size=mesh.nv), 0.0)
+    _both(contexts, mesh, mu, mask.astype(np.uint8), g, precision=precision)
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("n", [12, 34, 84])
 def test_right_hand_sides(contexts, n, precision):
     _increment(contexts, n, precision)
 
