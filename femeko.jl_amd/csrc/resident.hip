@@ -256,7 +256,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             // a brick's p stays in LDS; its elements past a run belong to the halo
             if (restart && (!BRICK || (j % TP) * BLOCK + tl < blen))
                 win[own_lds(j, tl)] = BRICK ? z[j] : p[BRICK ? 0 : j];
-            if (BRICK && j % TP == TP - 1) __builtin_amdgcn_sched_barrier(0);
+            if (BRICK && j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (!BRICK) {
 #pragma unroll
@@ -517,7 +517,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                         sol.store(0, row * A.us, A.u[at(row)] + inv_s * static_cast<double>(xj(j, tc)));
                         if constexpr (!BRICK) A.p[row] = p[j];
                     }
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
                 }
                 ++tag;
                 alive = all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
@@ -535,42 +535,81 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             }
             ++tag;
             s[0] = 0.0;
+            if (!GEN && act == 1) {
+                // all loads of two rows in flight together, without a branch: rows
+                // and neighbours that do not exist read zero
+                constexpr int Q = RPT > 1 ? 2 : 1;
+                const ValueColumns<double> val64(A.val64, A.K, A.ld), u64s(A.u, 1, n * A.us);
 #pragma unroll 1
-            for (int j = 0; j < RPT; ++j) {
-                const int32_t row = own_row(j, tc);
-                if (row >= n) continue;
-                const T dj = A.dinv[row];
-                double v = dj != T(0) ? A.r64[at(row)] : 0.0;
-                if (act == 1) {
-                    double y0 = 0.0, y1 = 0.0;
-                    if constexpr (GEN) {
-                        const int32_t sl = i0 / 64 + j * (BLOCK / 64) + wave, lane = tc & 63;
-                        const int64_t base = A.sptr[sl];
-                        const int32_t W = abs(A.swidth[sl]), ng = W >> 2;
-#pragma unroll 4
-                        for (int k = 0; k < W; ++k) {
-                            const int64_t e = base + (k < 4 * ng ? 4 * (64 * (k >> 2) + lane) + (k & 3)
-                                                                 : 256 * ng + 64 * (k - 4 * ng) + lane);
-                            const int32_t ix = A.sidx[e];
-                            y0 += A.val64[e] * A.u[at(ix < R ? i0 + ix : A.halo[h0 + ix - R])];
-                        }
-                    } else {
+                for (int j0 = 0; j0 < RPT; j0 += Q) {
+                    int32_t row[Q];
+                    double a[Q][2 * K], y[Q][2 * K], yc[Q], dg[Q], bv[Q];
+                    T dj[Q];
 #pragma unroll
-                        for (int k = 0; k < K; ++k)
-                            if (k < A.K) {
-                                const int32_t o = A.off[k], f = min(row + o, n - 1), bk = max(row - o, 0);
-                                const double *__restrict__ c = A.val64 + static_cast<int64_t>(k) * A.ld;
-                                const double vb64 = c[bk];
-                                y0 += c[row] * A.u[at(f)];  // 0 where row + o is past the last row
-                                y1 += (row >= o ? vb64 : 0.0) * A.u[at(bk)];
+                    for (int q = 0; q < Q; ++q) {
+                        row[q] = j0 + q < RPT ? own_row(j0 + q, tc) : kNoRow;
+                        const int32_t in = min(row[q], n - 1);
+                        row[q] = row[q] < n ? row[q] : kNoRow;
+                        const int32_t c = row[q] < n ? row[q] * A.us : kNoRow;
+#pragma unroll
+                        for (int k = 0; k < K; ++k) {
+                            a[q][k] = a[q][K + k] = y[q][k] = y[q][K + k] = 0.0;
+                            if (BRICK || k < A.K) {
+                                a[q][k] = val64.load(k, row[q]);
+                                a[q][K + k] = val64.load(k, row[q] - A.off[k]);
+                                y[q][k] = u64s.load(0, c + A.off[k] * A.us);
+                                y[q][K + k] = u64s.load(0, c - A.off[k] * A.us);
                             }
+                        }
+                        yc[q] = u64s.load(0, c);
+                        dg[q] = A.diag64[in];
+                        dj[q] = A.dinv[in];
+                        bv[q] = A.b ? A.b[in] : 0.0;
                     }
-                    const double y = (y0 + y1) + A.diag64[row] * A.u[at(row)];
-                    v = dj != T(0) ? (A.b ? A.b[row] - y : -y) : 0.0;
-                    A.r64[at(row)] = v;
-                    s[0] += v * v;
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        double y0 = 0.0, y1 = 0.0;
+#pragma unroll
+                        for (int k = 0; k < K; ++k) {
+                            y0 += a[q][k] * y[q][k];
+                            y1 += a[q][K + k] * y[q][K + k];
+                        }
+                        const double sum = (y0 + y1) + dg[q] * yc[q];
+                        const double v = dj[q] != T(0) && row[q] < n ? bv[q] - sum : 0.0;
+                        if (row[q] < n) A.r64[at(row[q])] = v;
+                        s[0] += v * v;
+                        rows.store(tag, row[q], dj[q] * static_cast<T>(A.s * v));
+                    }
                 }
-                rows.store(tag, row, dj * static_cast<T>(A.s * v));
+            } else {
+#pragma unroll 1
+                for (int j = 0; j < RPT; ++j) {
+                    const int32_t row = own_row(j, tc);
+                    if (row >= n) continue;
+                    const T dj = A.dinv[row];
+                    double v = dj != T(0) ? A.r64[at(row)] : 0.0;
+                    if constexpr (GEN) {
+                        if (act == 1) {
+                            double y0 = 0.0;
+                            const int32_t sl = i0 / 64 + j * (BLOCK / 64) + wave, lane = tc & 63;
+                            const int64_t base = A.sptr[sl];
+                            const int32_t W = abs(A.swidth[sl]), ng = W >> 2;
+#pragma unroll 4
+                            for (int k = 0; k < W; ++k) {
+                                const int64_t e = base + (k < 4 * ng ? 4 * (64 * (k >> 2) + lane) + (k & 3)
+                                                                     : 256 * ng + 64 * (k - 4 * ng) + lane);
+                                const int32_t ix = A.sidx[e];
+                                y0 += A.val64[e] * A.u[at(ix < R ? i0 + ix : A.halo[h0 + ix - R])];
+                            }
+                            const double y = y0 + A.diag64[row] * A.u[at(row)];
+                            v = dj != T(0) ? (A.b ? A.b[row] - y : -y) : 0.0;
+                            A.r64[at(row)] = v;
+                            s[0] += v * v;
+                        }
+                    }
+                    rows.store(tag, row, dj * static_cast<T>(A.s * v));
+                }
             }
             alive = alive && all_reduce5<BLOCK>(s, A.slots, me, A.nb, tag, sh);
             if (!alive) {
