@@ -778,7 +778,7 @@ template <typename T, int BLOCK, int RPT, int NK, bool REFINE = false, int NE = 
 static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     constexpr int R = BLOCK * RPT;
     constexpr int U = NE > 0   ? (RPT <= 2 ? 4 * RPT : 3 * RPT)
-                      : NE < 0 ? brick_halo<T>(NE < 0 ? RPT / -NE : 1, -NE)
+                      : NE < 0 ? brick_halo<T>(RPT / (NE < 0 ? -NE : 1), -NE)
                                : 2 * RPT + 2;
     const int most = std::min(m->ctx->num_cus, kMaxResidentBlocks);
     int nb = static_cast<int>((m->nv + R - 1) / R);
@@ -847,16 +847,18 @@ static int64_t rows_per_block(const fk_mesh *m) {
 // streamed one row ahead: the first shape of the list, by slots per thread,
 // whose threads, halo registers and LDS cover the mesh with one brick per CU.
 // The shapes are those that leave few slots empty on some mesh: an m^3 grid
-// wastes 1 to 20% of them. Measured per iteration (us; windows or, from the
-// second dash on, the three kernels in brackets), Kuhn meshes of n cells per side:
+// wastes 1 to 20% of them. Measured per iteration (us; in
+// brackets the windows or, for FP64 n > 100 and FP32 n > 126, the three kernels),
+// Kuhn meshes of n cells per side:
 //   FP64  n = 80  8.8 (10.9)   n = 90 11.6 (14.1)   n = 95 11.7 (18.5)   n = 100 13.7 (22.2)
 //         n = 105 16 (41.5)    n = 118 21 (52.7)    n = 125 24 (60.0)    n = 130 35 (67.5)
-//   FP32  n = 80  7.7 (8.7)    n = 95 9.3 (11.5)    n = 100 11.0 (13.5)  n = 115 14.3 (20.5)
-//         n = 126 17 (28.8)    n = 140 23.6 (45.6)  n = 150 27 (53.8)    n = 160 31.7 (61.8)
+//   FP32  n = 80  7.5 (8.7)    n = 95 9 (11.5)      n = 100 10.6 (13.5)  n = 118 14.0 (20.5)
+//         n = 126 16.3 (28.8)  n = 140 21.6 (45.6)  n = 150 25 (53.8)    n = 160 29.0 (61.8)
 // More rows in flight (2 or 3 per thread) were no faster at any size: n = 160
 // 40.0 us with 3, where they spill, n = 115 14.9 with 2 or 3. What bounds the
-// larger ones is the value stream from the MALL (7 columns, 117 MB at n = 160
-// in about 25 of the 31.7 us), then the exchange and the all-reduce (6 to 8).
+// larger ones is the value stream from the MALL: of 29.0 us at n = 160, 12.3 go
+// away when the values (7 columns, 117 MB) are not loaded and 3.0 without the
+// exchange; 3.2 are the residual replacements, one in 63 iterations.
 //
 // Up to four rows per thread the windows, which keep the values in registers,
 // are faster: FP64 n = 76 7.1 us against 7.8, n = 70 6.3 against 7.9.
@@ -890,6 +892,7 @@ static bool launch_bricks(fk_mesh *m, ResidentArgs<float> &A) {
 //   n = 79  512 x 4   7.6 (26.9)     n = 85  512 x 5  11.3 (29.4)
 //   n = 90  512 x 6  14.5 (31.5)     n = 95  512 x 7  17.8 (34)
 //   n = 100 512 x 8  21.8 (36.8)
+// The last four shapes serve stencils that are cut into no bricks.
 // One shape up costs: n = 63 on 512 x 3 5.8, n = 79 on 512 x 5 10.9, n = 85 on
 // 512 x 6 13.6. More rows than 256 blocks of 4096 keep the three-kernel
 // iteration: the windows of more rows per block exceed the LDS.
@@ -913,6 +916,7 @@ static bool launch_by_rows(fk_mesh *m, ResidentArgs<double> &A) {
 //   n = 63  512 x 2   5.2 (19.0)     n = 75  512 x 4   6.9 (20.7)
 //   n = 90 1024 x 3   9.7 (22.8)     n = 100 512 x 8  13.7 (25.2)
 //   n = 115 512 x 12 20   (31)       n = 126 512 x 16 28.1 (35.6)
+// The last four shapes serve stencils that are cut into no bricks.
 static bool launch_by_rows(fk_mesh *m, ResidentArgs<float> &A) {
     const int64_t per = rows_per_block(m);
     if (per > kBrickRows && launch_bricks(m, A)) return true;
