@@ -165,7 +165,10 @@ int fk_lagrange(fk_mesh *mesh, double *C);
 int fk_set_dirichlet(fk_mesh *mesh, const uint8_t *mask, const double *g);
 /* Jacobi-preconditioned CG (the solver of magnetostatics.cpp:26-38 and
  * run.jl:141) on the assembled matrix, stopping at ||r||_2 < rtol ||b||_2.
- * precision FK_PREC_F64: one FP64 PCG to rtol.
+ * precision FK_PREC_F64: one FP64 PCG to rtol. A solve that runs as one
+ * resident launch and has iterated ends with a Jacobi step x + D^-1 r / 3 (it
+ * removes modes of sliver elements that rounding brings back), taken only
+ * where the residual after it is below the tolerance too.
  * precision FK_PREC_F32_REFINED: FP32 values and PCG recursion (difference-
  * form SpMV on the stencil and SELL copies); at the end of each chunk of iterations in
  * which the FP32 recursive residual has fallen by the factor inner_rtol
