@@ -92,6 +92,7 @@ struct CgState {
     // kernel reads a flag that a block of the same launch may be writing
     int32_t done_at[2];
     int32_t status;     // FK_OK, FK_ERR_NOT_CONVERGED, FK_ERR_SINGULAR
+    int32_t timed_out;  // resident launches: a wait of some block ran out
     int64_t iters;      // completed iterations
     double thresh;      // rtol^2 * ||b||^2
     double bb;          // ||b||^2

@@ -355,7 +355,8 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                     load_row(own_row((j + NK) % RPT, t), v[j % NK]);
                     const double zd = static_cast<double>(z[j]), qd = static_cast<double>(q);
                     const double rd = static_cast<double>(reciprocal(d[j]) * z[j]);
-                    s[0] += (last ? rd : static_cast<double>(d[j] != T(0) ? pj : T(0))) * qd;  // past a run: any LDS word
+                    // past a run pj is any LDS word
+                    s[0] += (last ? rd : static_cast<double>(d[j] != T(0) ? pj : T(0))) * qd;
                     s[1] += rd * zd;
                     s[2] += qd * (last ? qd : zd);
                     s[3] += qd * static_cast<double>(w[j]);
@@ -656,6 +657,10 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             }
         }
     }
+    // Block 0 may have seen the last round whole where another block gave up on
+    // it. A refined solve has stored u by then; x of FP64 differs by the step.
+    if (!REFINE && code == FK_ERR_HIP && tid == 0)
+        __hip_atomic_store(&A.state->timed_out, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (me == 0 && tid == 0) {
         if constexpr (REFINE) {
             A.ru->nrep = nrep;
@@ -697,10 +702,12 @@ __global__ __launch_bounds__(BLOCK) void k_resident_batch(const ResidentArgs<T> 
     resident_solve<T, BLOCK, RPT, NK, U, true, 0>(A, me, me * (BLOCK * RPT));
 }
 
-// slots, and the rows n..stride of the two exchange arrays
+// slots, the rows n..stride of the two exchange arrays and the time-out flag
 template <typename T>
-__global__ void k_resident_clear(u64 *__restrict__ slots, int words, T *__restrict__ w, int32_t n, int32_t stride) {
+__global__ void k_resident_clear(u64 *__restrict__ slots, int words, T *__restrict__ w, int32_t n, int32_t stride,
+                                 CgState *__restrict__ state) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    if (t == 0) state->timed_out = 0;
     for (int i = t; i < words; i += step) slots[i] = 0;
     for (int i = n + t; i < stride; i += step) w[i] = w[stride + i] = T(0);
 }
@@ -845,7 +852,7 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     auto kern = k_resident_pcg<T, BLOCK, RPT, NK, U, REFINE, NE>;
     FK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                static_cast<int>(lds)));
-    k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, reduce_words(nb), A.w, A.n, A.stride);
+    k_resident_clear<T><<<64, 256, 0, st>>>(A.slots, reduce_words(nb), A.w, A.n, A.stride, A.state);
     FK_HIP(hipGetLastError());
     void *args[] = {&A};
     const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kern), dim3(nb), dim3(BLOCK),
@@ -1139,7 +1146,8 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
     CgState *hs = m->hstate.ptr;
     FK_HIP(hipMemcpyAsync(hs, w.state.get(), sizeof(CgState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
-    if (hs->status == FK_ERR_HIP) return false;  // a wait ran out (another process's launch); r0 is unchanged
+    // a wait ran out (another process's launch); r0 is unchanged
+    if (hs->status == FK_ERR_HIP || hs->timed_out) return false;
     *out = *hs;
     return true;
 }
