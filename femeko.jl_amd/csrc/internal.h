@@ -169,11 +169,12 @@ namespace fk {
 // Copies to pageable memory through a ring of pinned chunks that several
 // threads empty (transfer.hip); one copy at a time, made with the first one.
 struct HostLink {
-    explicit HostLink(int device);
+    static std::unique_ptr<HostLink> make(int device);  // null without the pinned memory or the events
     ~HostLink();
     void copy(void *to, const void *from, size_t bytes, hipStream_t st);  // returns when `to` holds the data
 
   private:
+    explicit HostLink(int dev) : device(dev) {}
     void work(int t);
     void share(int t);
     hipError_t issue(size_t chunk);
@@ -189,7 +190,7 @@ struct HostLink {
     char *dst = nullptr;
     const char *src = nullptr;
     size_t bytes = 0, piece = 0;
-    int takers = 1;
+    int most = 1, takers = 1;  // threads that empty the ring: at most, and of this copy
     hipStream_t stream = nullptr;
     hipError_t error = hipSuccess;
 };
@@ -204,6 +205,7 @@ struct fk_context {
     std::string err;
     fk::TimingEvents timing;
     std::unique_ptr<fk::HostLink> link;
+    bool no_link = false;  // it could not be made: plain copies from then on
 };
 
 struct fk_mesh {

@@ -6,6 +6,7 @@
 // ring of pinned chunks and several threads empty it, so that faults and copies
 // overlap with one another and with the transfer.
 #include <cstring>
+#include <system_error>
 
 #include "internal.h"
 
@@ -21,14 +22,27 @@ constexpr int kThreads = 8, kSlots = 2 * kThreads;
 constexpr size_t kChunk = 2 << 20, kPiece = 1 << 20, kLong = 16 << 20;
 constexpr size_t kLinkMin = 512 << 10, kLinkMany = 2 << 20;
 
-HostLink::HostLink(int dev) : device(dev) {
-    ring.alloc(kSlots * kChunk);
-    for (int i = 0; i < kSlots; ++i) {
-        hipEvent_t e = nullptr;
-        FK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        ev.push_back(e);
+std::unique_ptr<HostLink> HostLink::make(int device) {
+    try {
+        std::unique_ptr<HostLink> l(new HostLink(device));
+        l->ring.alloc(kSlots * kChunk);
+        l->ev.reserve(kSlots);
+        for (int i = 0; i < kSlots; ++i) {
+            hipEvent_t e = nullptr;
+            FK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            l->ev.push_back(e);
+        }
+        l->threads.reserve(kThreads);
+        try {
+            for (int t = 1; t < kThreads; ++t) l->threads.emplace_back([p = l.get(), t] { p->work(t); });
+        } catch (const std::system_error &) {  // no more threads: those there are, the caller's at least
+        }
+        while (2 * l->most <= static_cast<int>(l->threads.size()) + 1) l->most *= 2;
+        return l;
+    } catch (...) {
+        (void)hipGetLastError();
+        return nullptr;
     }
-    for (int t = 1; t < kThreads; ++t) threads.emplace_back([this, t] { work(t); });
 }
 
 HostLink::~HostLink() {
@@ -51,7 +65,7 @@ void HostLink::work(int t) {
             if (quit) return;
             seen = job;
         }
-        share(t);
+        if (t < takers) share(t);
         const std::lock_guard<std::mutex> l(mu);
         if (--left == 0) done.notify_one();
     }
@@ -90,7 +104,7 @@ void HostLink::copy(void *to, const void *from, size_t n, hipStream_t st) {
     stream = st;
     error = hipSuccess;
     piece = n < kLong ? kPiece : kChunk;
-    takers = n < kLinkMany ? 1 : kThreads;
+    takers = n < kLinkMany ? 1 : most;
     for (int c = 0; c < kSlots && c * piece < n; ++c) FK_HIP(issue(c));
     if (takers > 1) {
         const std::lock_guard<std::mutex> l(mu);
@@ -111,9 +125,12 @@ void copy_out(fk_context *ctx, void *to, const void *from, size_t bytes) {
         const hipError_t e = hipPointerGetAttributes(&a, to);
         if (e != hipSuccess) (void)hipGetLastError();
         if (e != hipSuccess || a.type == hipMemoryTypeUnregistered) {
-            if (!ctx->link) ctx->link = std::make_unique<HostLink>(ctx->device);
-            ctx->link->copy(to, from, bytes, st);
-            return;
+            if (!ctx->link && !ctx->no_link) ctx->link = HostLink::make(ctx->device);
+            ctx->no_link = !ctx->link;
+            if (ctx->link) {
+                ctx->link->copy(to, from, bytes, st);
+                return;
+            }
         }
     }
     FK_HIP(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, st));
