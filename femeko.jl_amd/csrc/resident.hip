@@ -35,13 +35,13 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
-#include <thread>
 #include <utility>
 #include <vector>
 
 #include "device.h"
 #include "internal.h"
 #include "resident.h"
+#include "resident_lists.h"
 
 namespace fk {
 
@@ -799,6 +799,19 @@ static bool place_bricks(const int32_t *off, int K, int64_t n, int most, int BZ,
     return true;
 }
 
+// Scratch that the three kernels do without: false where there is no memory for it.
+template <typename F>
+static bool have_memory(F reserve) {
+    try {
+        reserve();
+        return true;
+    } catch (const Error &e) {
+        if (e.code != FK_ERR_OOM) throw;
+        (void)hipGetLastError();
+        return false;
+    }
+}
+
 // halo elements per thread of a brick at most: its two outer planes, and the
 // ends of the inner ones up to a reach of 170 (FP64: 128)
 template <typename T>
@@ -844,8 +857,11 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     const int64_t reach = NE < 0 ? m->nv : static_cast<int64_t>(nb) * R + (NE > 0 ? 0 : m->st_off[m->st_K - 1] + R);
     const int64_t stride = (reach + 63) / 64 * 64;
     hipStream_t st = m->ctx->stream;
-    m->res_slots.ensure(reduce_words(kMaxResidentBlocks));
-    m->res_w.ensure(static_cast<size_t>(2 * stride));
+    if (!have_memory([&] {
+            m->res_slots.ensure(reduce_words(kMaxResidentBlocks));
+            m->res_w.ensure(static_cast<size_t>(2 * stride));
+        }))
+        return false;
     A.stride = static_cast<int32_t>(stride);
     A.slots = m->res_slots.get();
     A.w = reinterpret_cast<T *>(m->res_w.get());
@@ -1015,104 +1031,39 @@ static bool launch_sell(fk_mesh *m, ResidentArgs<float> &A) {
     }
 }
 
-// The LDS index of every SELL entry and the halo list of every block, from the
-// host's copy of the pattern while build_sell holds it. A block's halo is the
-// sorted set of the columns its rows have outside the block; on renumbered
-// meshes it is 2.2 to 2.5 times the block's rows. No lists are made (res_R = 0)
-// where the mesh is too large or its rows too long for the resident launch.
+// The lists of resident_lists.h on the device. No lists (res_R = 0: the three
+// kernels) where the mesh is too large or its rows too long for the resident
+// launch, or where the lists cannot be had: the solves do not need them.
 void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::vector<int32_t> &ci,
                          const std::vector<int32_t> &width, const std::vector<std::vector<int32_t>> &shared,
                          const std::vector<int64_t> &vptr) {
     m->res_R = 0;
-    const int64_t nv = m->nv, ns = static_cast<int64_t>(width.size());
     int32_t most = 0;
     for (int32_t w : width) most = std::max(most, w < 0 ? -w : w);
     const int R = sell_rows_per_block(m, most);
     if (!R || most == 0) return;
-    const int nb = static_cast<int>((nv + R - 1) / R);
-    std::vector<std::vector<int32_t>> halo(static_cast<size_t>(nb));
-    std::vector<uint16_t> idx(static_cast<size_t>(vptr[ns]));
-    const int nth = static_cast<int>(std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency())));
-    std::vector<std::thread> th;
-    bool fits = true;
-    std::mutex mu;
-    for (int q = 0; q < nth; ++q)
-        th.emplace_back([&, q] {
-            std::vector<int32_t> place(static_cast<size_t>(nv), -1);  // halo position of a row of the block at hand
-            for (int b = nb * q / nth; b < nb * (q + 1) / nth; ++b) {
-                const int64_t r0 = static_cast<int64_t>(b) * R, r1 = std::min(nv, r0 + R);
-                std::vector<int32_t> &h = halo[b];
-                for (int64_t k = rp[r0]; k < rp[r1]; ++k) {
-                    const int32_t c = ci[k];
-                    if ((c < r0 || c >= r1) && place[c] < 0) {
-                        place[c] = 0;
-                        h.push_back(c);
-                    }
-                }
-                std::sort(h.begin(), h.end());
-                if (h.size() + R > 0xfffe) {
-                    const std::lock_guard<std::mutex> lock(mu);
-                    fits = false;
-                    return;
-                }
-                for (size_t e = 0; e < h.size(); ++e) place[h[e]] = static_cast<int32_t>(e);
-                auto at = [&](int64_t c) {
-                    return static_cast<uint16_t>(c >= r0 && c < r1 ? c - r0 : R + place[c]);
-                };
-                for (int64_t s = r0 / 64; s < std::min(ns, (r0 + R) / 64); ++s) {
-                    const int32_t W = width[s] < 0 ? -width[s] : width[s], ng = W >> 2;
-                    for (int lane = 0; lane < 64; ++lane) {
-                        const int64_t r = s * 64 + lane;
-                        const uint16_t own = static_cast<uint16_t>(r - r0);
-                        const int32_t *lo = r < nv ? ci.data() + rp[r] : nullptr;
-                        const int32_t *hi = r < nv ? ci.data() + rp[r + 1] : nullptr;
-                        int32_t k = 0;
-                        auto put = [&](uint16_t v) {
-                            const int64_t o = k < 4 * ng ? 4 * (64 * static_cast<int64_t>(k >> 2) + lane) + (k & 3)
-                                                         : 256 * static_cast<int64_t>(ng) + 64 * (k - 4 * ng) + lane;
-                            idx[vptr[s] + o] = v;
-                            ++k;
-                        };
-                        if (width[s] < 0) {
-                            for (int32_t off : shared[s]) {
-                                const int64_t c = r + off;
-                                const int32_t *f = r < nv && c >= 0 && c < nv
-                                                       ? std::lower_bound(lo, hi, static_cast<int32_t>(c))
-                                                       : hi;
-                                put(f != hi && *f == c ? at(c) : own);
-                            }
-                        } else {
-                            for (const int32_t *c = lo; c != hi; ++c)
-                                if (*c != r) put(at(*c));
-                            while (k < W) put(own);
-                        }
-                    }
-                }
-                for (int32_t c : h) place[c] = -1;
-            }
-        });
-    for (auto &t : th) t.join();
-    if (!fits) return;
-    std::vector<int32_t> ptr(static_cast<size_t>(nb) + 1, 0), list;
-    int32_t hmax = 0;
-    for (int b = 0; b < nb; ++b) {
-        ptr[b + 1] = ptr[b] + static_cast<int32_t>(halo[b].size());
-        hmax = std::max(hmax, static_cast<int32_t>(halo[b].size()));
-        list.insert(list.end(), halo[b].begin(), halo[b].end());
+    try {
+        ResidentLists l;
+        if (!resident_lists(m->nv, R, rp, ci, width, shared, vptr, l)) return;
+        m->res_sidx.alloc(l.idx.size());
+        m->res_halo_ptr.alloc(l.ptr.size());
+        m->res_halo.alloc(std::max<size_t>(l.halo.size(), 1));
+        hipStream_t st = m->ctx->stream;
+        const auto send = [&](auto &to, const auto &from) {
+            FK_HIP(hipMemcpyAsync(to.get(), from.data(), from.size() * sizeof(from[0]), hipMemcpyHostToDevice, st));
+        };
+        send(m->res_sidx, l.idx);
+        send(m->res_halo_ptr, l.ptr);
+        if (!l.halo.empty()) send(m->res_halo, l.halo);
+        FK_HIP(hipStreamSynchronize(st));
+        m->res_R = R;
+        m->res_width = most;
+        m->res_halo_max = l.halo_max;
+    } catch (const Error &e) {
+        if (e.code != FK_ERR_OOM) throw;
+        (void)hipGetLastError();
+    } catch (const std::bad_alloc &) {
     }
-    hipStream_t st = m->ctx->stream;
-    m->res_sidx.alloc(idx.size());
-    m->res_halo_ptr.alloc(ptr.size());
-    m->res_halo.alloc(std::max<size_t>(list.size(), 1));
-    FK_HIP(hipMemcpyAsync(m->res_sidx.get(), idx.data(), idx.size() * sizeof(uint16_t), hipMemcpyHostToDevice, st));
-    FK_HIP(hipMemcpyAsync(m->res_halo_ptr.get(), ptr.data(), ptr.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    if (!list.empty())
-        FK_HIP(hipMemcpyAsync(m->res_halo.get(), list.data(), list.size() * sizeof(int32_t), hipMemcpyHostToDevice,
-                              st));
-    FK_HIP(hipStreamSynchronize(st));
-    m->res_R = R;
-    m->res_width = most;
-    m->res_halo_max = hmax;
 }
 
 // the copy of the matrix a resident launch can run on, with fresh values
@@ -1265,11 +1216,17 @@ static bool launch_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sy
         for (int b = 0; b < args[s].nb; ++b) rounds[k].push_back(make_int2(s, b));
     }
     if (rounds.size() > most) return false;
-    B.words.ensure(words);
-    B.w.ensure(floats);
-    B.args.ensure(S * sizeof(ResidentArgs<float>));
-    B.state.ensure(S);
-    B.ru.ensure(S);
+    std::vector<int2> table;
+    for (const auto &r : rounds) table.insert(table.end(), r.begin(), r.end());
+    if (!have_memory([&] {
+            B.words.ensure(words);
+            B.w.ensure(floats);
+            B.args.ensure(S * sizeof(ResidentArgs<float>));
+            B.state.ensure(S);
+            B.ru.ensure(S);
+            B.table.ensure(table.size());
+        }))
+        return false;
     words = floats = 0;
     for (int s = 0; s < S; ++s) {
         const ResidentSystem &q = sys[s];
@@ -1298,9 +1255,6 @@ static bool launch_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sy
         words += reduce_words(A.nb);
         floats += 2 * static_cast<int64_t>(A.stride);
     }
-    std::vector<int2> table;
-    for (const auto &r : rounds) table.insert(table.end(), r.begin(), r.end());
-    B.table.ensure(table.size());
     FK_HIP(hipMemcpyAsync(B.args.get(), args.data(), S * sizeof(ResidentArgs<float>), hipMemcpyHostToDevice, st));
     FK_HIP(hipMemcpyAsync(B.table.get(), table.data(), table.size() * sizeof(int2), hipMemcpyHostToDevice, st));
     k_resident_zero<<<256, 256, 0, st>>>(B.words.get(), words, B.w.get(), floats);
