@@ -387,7 +387,7 @@ void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::
                          const std::vector<int64_t> &vptr);
 // the same for the FP32 recursion with FP64 residual replacement
 bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
-                      int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status);
+                      int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status, bool *started);
 CgState run_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref);
 int solve_f32_increment(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, int64_t *iters);
 int solve_f32_free(fk_mesh *m, double *u, const double *b, double rtol, int64_t max_iter, double bb_ref,

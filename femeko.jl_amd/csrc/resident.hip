@@ -1105,9 +1105,10 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
 
 // The FP32-refined solve of solve.hip's solve_f32_replace from the FP64
 // residual in r64 (its norm^2 rr): false when this mesh or moment does not
-// allow a resident launch; u and r64 may then have changed.
+// allow a resident launch; u and r64 may then have changed if one was started.
 bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
-                      int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status) {
+                      int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status, bool *started) {
+    *started = false;
     if (!resident_kind(m)) return false;
     const bool stencil = m->kind == FK_SPMV_STENCIL;
     PcgWork<float> &w = m->w32;
@@ -1138,6 +1139,7 @@ bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double 
     A.G = chunk;
     const std::lock_guard<std::mutex> alone(resident_mutex(m->ctx->device));
     if (!(stencil ? launch_by_rows(m, A) : launch_sell(m, A))) return false;
+    *started = true;
     hipStream_t st = m->ctx->stream;
     CgState *hs = m->hstate.ptr;
     RuState *hr = m->hru.ptr;

@@ -1893,8 +1893,10 @@ static int solve_f32_replace(fk_mesh *m, double *u, const double *b, double rtol
     sync_solver_values<float>(m);
     if (std::isfinite(rr)) {
         int status = FK_OK;
-        if (resident_refined(m, u, b, rr, thresh, delta, max_iter, G, iters, nrep, rr_out, &status)) return status;
-        rr = neg_residual(m, u, m->r64.get(), b);
+        bool started = false;
+        if (resident_refined(m, u, b, rr, thresh, delta, max_iter, G, iters, nrep, rr_out, &status, &started))
+            return status;
+        if (started) rr = neg_residual(m, u, m->r64.get(), b);
     }
     const double s = 1.0 / std::sqrt(rr);
     const double target2 = thresh * s * s;
