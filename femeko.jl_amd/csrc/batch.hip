@@ -1360,7 +1360,8 @@ static bool batch_solve_resident(fk_batch *b, double delta, int64_t max_iter, co
                                  const std::vector<double> &scale, const std::vector<double> &th,
                                  const std::vector<double> &t2, std::vector<int64_t> &its, std::vector<int32_t> &nrep,
                                  std::vector<int32_t> &fst, std::vector<double> &rr64) {
-    if (b->ctx->timing.enabled || b->stencil != 1 || !b->st_valid) return false;
+    b->res.rows = b->res.launches = 0;
+    if (b->ctx->timing.enabled || !b->ctx->resident || b->stencil != 1 || !b->st_valid) return false;
     fk_mesh *m = b->mesh;
     const int nr = b->nrhs;
     std::vector<ResidentSystem> sys;
@@ -1974,6 +1975,13 @@ int fk_batch_set_format(fk_batch *b, int32_t format) {
 int fk_batch_solver_format(fk_batch *b, int32_t *format) {
     if (!b || !format) return FK_ERR_INVALID_ARG;
     *format = b->stencil < 0 ? -1 : (b->stencil == 1 ? FK_SPMV_STENCIL : FK_SPMV_CSR);
+    return FK_OK;
+}
+
+int fk_batch_solve_launch(fk_batch *b, int32_t *rows_per_block, int32_t *launches) {
+    if (!b) return FK_ERR_INVALID_ARG;
+    if (rows_per_block) *rows_per_block = b->res.rows;
+    if (launches) *launches = b->res.launches;
     return FK_OK;
 }
 

@@ -201,6 +201,7 @@ struct fk_context {
     hipStream_t stream = nullptr;
     int num_cus = 256;
     bool graphs = true;  // capture PCG iteration chunks in hipGraphs (FEMEKO_HIP_GRAPHS=0 disables)
+    bool resident = true;  // solves in one resident launch where the mesh fits (FEMEKO_HIP_RESIDENT=0 disables)
     bool one_shot = false;  // destroyed by the call that made it: no copy threads
     std::string err;
     fk::TimingEvents timing;
@@ -335,6 +336,8 @@ struct fk_mesh {
     int32_t res_R = 0, res_width = 0, res_halo_max = 0;
     fk::DevBuf<uint16_t> res_sidx;
     fk::DevBuf<int32_t> res_halo_ptr, res_halo;
+    // how the last solve that iterated ran (FK_SOLVE_*; -1: none yet), rows per block, blocks
+    int32_t launch_layout = -1, launch_rows = 0, launch_blocks = 0;
 
     fk::PcgWork<double> w64;
     fk::PcgWork<float> w32;
@@ -408,6 +411,7 @@ struct ResidentSystem {
 struct ResidentBatch {
     fk_context *ctx = nullptr;
     bool started = false;  // the last call changed u and r64
+    int32_t rows = 0, launches = 0;  // rows per block and launches of the last call
     DevBuf<unsigned long long> words;
     DevBuf<float> w;
     DevBuf<char> args;

@@ -370,6 +370,8 @@ int fk_context_create(int device, fk_context **out) {
         const char *tool = std::getenv("ROCP_TOOL_LIBRARIES");
         const bool profiled = tool && tool[0] != '\0';
         ctx->graphs = g ? g[0] != '0' : !profiled;
+        const char *r = std::getenv("FEMEKO_HIP_RESIDENT");
+        ctx->resident = !(r && r[0] == '0');
         FK_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
         fk::noalloc_setup(device);
     } catch (const fk::Error &e) {

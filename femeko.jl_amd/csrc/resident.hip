@@ -878,6 +878,9 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
         return false;
     }
     FK_HIP(e);
+    m->launch_layout = NE < 0 ? FK_SOLVE_BRICKS : NE > 0 ? FK_SOLVE_SELL : FK_SOLVE_WINDOWS;
+    m->launch_rows = R;
+    m->launch_blocks = nb;
     return true;
 }
 
@@ -1068,7 +1071,7 @@ void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::
 
 // the copy of the matrix a resident launch can run on, with fresh values
 static bool resident_kind(const fk_mesh *m) {
-    if (m->ctx->timing.enabled) return false;
+    if (m->ctx->timing.enabled || !m->ctx->resident) return false;
     if (m->kind == FK_SPMV_STENCIL) return m->st_K <= kResK;
     return m->kind == FK_SPMV_SELL64 && m->format != FK_SPMV_CSR && m->have_sell && m->res_R > 0;
 }
@@ -1278,11 +1281,14 @@ static bool launch_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sy
         at += r.size();
     }
     FK_HIP(hipStreamSynchronize(st));  // args and table go out of scope
+    B.rows = R;
+    B.launches = static_cast<int32_t>(rounds.size());
     return true;
 }
 
 bool resident_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sys, double delta, int64_t max_iter, int chunk,
                     std::vector<CgState> &state, std::vector<RuState> &ru) {
+    B.rows = B.launches = 0;
     if (sys.empty()) return true;
     const std::lock_guard<std::mutex> alone(resident_mutex(B.ctx->device));
     B.started = false;
@@ -1298,7 +1304,10 @@ bool resident_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sys, do
     FK_HIP(hipMemcpyAsync(ru.data(), B.ru.get(), S * sizeof(RuState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
     for (const RuState &r : ru)
-        if (r.status == FK_ERR_HIP) return false;  // a wait ran out (another process's launch)
+        if (r.status == FK_ERR_HIP) {  // a wait ran out (another process's launch)
+            B.rows = B.launches = 0;
+            return false;
+        }
     return true;
 }
 

@@ -1633,6 +1633,11 @@ static void harvest_timing(fk_context *ctx, int64_t valid) {
     te.used = 0;
 }
 
+static void three_kernels(fk_mesh *m) {
+    m->launch_layout = FK_SOLVE_KERNELS;
+    m->launch_rows = m->launch_blocks = 0;
+}
+
 // PCG on work<T>: r holds the initial residual on entry; x returns the
 // correction. bb_ref < 0: tolerance relative to ||r0||, else to sqrt(bb_ref).
 template <typename T>
@@ -1645,6 +1650,7 @@ static CgState run_pcg(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref)
         CgState done{};
         if (resident_pcg_f64(m, rtol, max_iter, bb_ref, &done)) return done;
     }
+    three_kernels(m);
     k_cg_init<T><<<nb, kBlock, 0, st>>>(w.x.get(), w.r.get(), w.p.get(), w.dinv.get(), w.part_rz.get(),
                                         w.part_bb.get(), m->nv, m->chunk, nb);
     k_cg_start<<<1, kBlock, 0, st>>>(w.part_bb.get(), nb, bb_ref, rtol, max_iter, w.state.get());
@@ -1898,6 +1904,7 @@ static int solve_f32_replace(fk_mesh *m, double *u, const double *b, double rtol
             return status;
         if (started) rr = neg_residual(m, u, m->r64.get(), b);
     }
+    three_kernels(m);
     const double s = 1.0 / std::sqrt(rr);
     const double target2 = thresh * s * s;
     k_scale_to_f32<<<grid_for(nv, 256), 256, 0, st>>>(m->r64.get(), w.r.get(), s, nv);
@@ -2522,6 +2529,14 @@ int fk_solver_format(fk_mesh *m, int32_t *format, int32_t *stencil_offsets, int3
         if (offsets && *format == FK_SPMV_STENCIL)
             for (int k = 0; k < m->st_K; ++k) offsets[k] = m->st_off[k];
     });
+}
+
+int fk_solve_launch(fk_mesh *m, int32_t *layout, int32_t *rows_per_block, int32_t *blocks) {
+    if (!m || !layout) return FK_ERR_INVALID_ARG;
+    *layout = m->launch_layout;
+    if (rows_per_block) *rows_per_block = m->launch_rows;
+    if (blocks) *blocks = m->launch_blocks;
+    return FK_OK;
 }
 
 int fk_sell_info(fk_mesh *m, int64_t *nslices, int64_t *shared_slices, int64_t *entries) {

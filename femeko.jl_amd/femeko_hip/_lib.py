@@ -80,6 +80,7 @@ SIGNATURES = {
     "fk_solve": (_c.c_int, [_vp, _c.c_int32, _c.c_double, _c.c_int64, _c.c_double, _c.c_int32, _c.c_int32,
                             _i64p, _ip, _dp]),
     "fk_solve_rhs": (_c.c_int, [_vp, _dp, _c.c_double, _c.c_int64, _dp, _i64p, _dp]),
+    "fk_solve_launch": (_c.c_int, [_vp, _ip, _ip, _ip]),
     "fk_potential": (_c.c_int, [_vp, _dp]),
     "fk_set_potential": (_c.c_int, [_vp, _dp]),
     "fk_field": (_c.c_int, [_vp, _dp, _dp, _dp]),
@@ -113,6 +114,7 @@ SIGNATURES = {
     "fk_batch_set_precision": (_c.c_int, [_vp, _c.c_int32]),
     "fk_batch_set_format": (_c.c_int, [_vp, _c.c_int32]),
     "fk_batch_solver_format": (_c.c_int, [_vp, _c.POINTER(_c.c_int32)]),
+    "fk_batch_solve_launch": (_c.c_int, [_vp, _ip, _ip]),
     "fk_batch_set_launch": (_c.c_int, [_vp, _c.c_int32, _c.c_int32]),
     "fk_batch_launch": (_c.c_int, [_vp, _ip, _ip, _ip, _ip]),
     "fk_set_timing": (_c.c_int, [_vp, _c.c_int32]),

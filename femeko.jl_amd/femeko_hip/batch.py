@@ -106,6 +106,14 @@ class Batch:
         sh = (self.nmesh, self.nrhs)
         return BatchReport(it.reshape(sh), outer.reshape(sh), rel.reshape(sh))
 
+    def solve_launch(self):
+        """(rows per block, launches) of the last solve's resident launches,
+        (0, 0) where it ran on the three kernels per iteration."""
+        r, n = ctypes.c_int32(0), ctypes.c_int32(0)
+        self.ctx.check(self._L.fk_batch_solve_launch(self.handle, ctypes.byref(r), ctypes.byref(n)),
+                       "fk_batch_solve_launch")
+        return r.value, n.value
+
     def potential(self, m: int) -> np.ndarray:
         """(nrhs, nv[m]) potentials of mesh m."""
         out = np.empty(self.nrhs * int(self.nv[m]))

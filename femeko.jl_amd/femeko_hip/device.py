@@ -444,6 +444,15 @@ class DeviceMesh:
         name = {0: "csr", 1: "sell64", 3: "stencil"}[int(f.value)]
         return name, tuple(int(offs[i]) for i in range(int(k.value)))
 
+    def solve_launch(self):
+        """(layout, rows per block, blocks) of the last solve that iterated:
+        'kernels' (three per iteration; 0, 0), 'windows', 'bricks' or 'sell'
+        (one resident launch); None before the first."""
+        v = [ctypes.c_int32(0) for _ in range(3)]
+        self.ctx.check(self._L.fk_solve_launch(self.handle, *[ctypes.byref(x) for x in v]), "fk_solve_launch")
+        name = {-1: None, 0: "kernels", 1: "windows", 2: "bricks", 3: "sell"}[v[0].value]
+        return name, v[1].value, v[2].value
+
     def sell_info(self):
         """(slices, shared-offset slices, stored entries) of the SELL copy."""
         a, b, c = ctypes.c_int64(0), ctypes.c_int64(0), ctypes.c_int64(0)

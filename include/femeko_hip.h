@@ -194,6 +194,19 @@ int fk_solve(fk_mesh *mesh, int32_t precision, double rtol, int64_t max_iter, do
  * and adjoint solves. */
 int fk_solve_rhs(fk_mesh *mesh, const double *b, double rtol, int64_t max_iter, double *x,
                  int64_t *iterations, double *relres);
+/* How the last solve on the mesh that iterated ran (fk_solve and the solves
+ * inside the calls below): *layout FK_SOLVE_KERNELS (three kernels per
+ * iteration) or the layout of its one resident launch, with its rows per block
+ * and blocks (0 with the three kernels); -1 before the first. One resident
+ * launch runs at a time on a device: those of several contexts of a process
+ * take turns, and a launch that finds the device held by another process ends
+ * by itself and its solve runs on the three kernels. FEMEKO_HIP_RESIDENT=0 in
+ * the environment when a context is created keeps it to the three kernels. */
+#define FK_SOLVE_KERNELS 0
+#define FK_SOLVE_WINDOWS 1     /* stencil copy, a block's rows consecutive */
+#define FK_SOLVE_BRICKS 2      /* stencil copy of a grid of boxes, rows of a few planes */
+#define FK_SOLVE_SELL 3        /* SELL copy */
+int fk_solve_launch(fk_mesh *mesh, int32_t *layout, int32_t *rows_per_block, int32_t *blocks);
 int fk_potential(fk_mesh *mesh, double *phi);
 int fk_set_potential(fk_mesh *mesh, const double *phi);
 
@@ -398,6 +411,9 @@ int fk_batch_set_format(fk_batch *batch, int32_t format);
 /* The SpMM copy in use: FK_SPMV_CSR or FK_SPMV_STENCIL, or -1 before the
  * first solve or autotune. */
 int fk_batch_solver_format(fk_batch *batch, int32_t *format);
+/* Rows per block and number of the resident launches that held the last
+ * solve's systems, 0 and 0 where it ran on the three kernels per iteration. */
+int fk_batch_solve_launch(fk_batch *batch, int32_t *rows_per_block, int32_t *launches);
 /* phi: nrhs * nv[mesh], right-hand side major */
 int fk_batch_potential(fk_batch *batch, int32_t mesh, double *phi);
 /* Autotuner: times the batched SpMM on this batch (all systems active) and
