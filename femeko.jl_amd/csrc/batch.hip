@@ -1361,7 +1361,7 @@ static bool batch_solve_resident(fk_batch *b, double delta, int64_t max_iter, co
                                  const std::vector<double> &t2, std::vector<int64_t> &its, std::vector<int32_t> &nrep,
                                  std::vector<int32_t> &fst, std::vector<double> &rr64) {
     b->res.rows = b->res.launches = 0;
-    if (b->ctx->timing.enabled || !b->ctx->resident || b->stencil != 1 || !b->st_valid) return false;
+    if (b->stencil != 1 || !b->st_valid || !resident_allowed(b->ctx)) return false;
     fk_mesh *m = b->mesh;
     const int nr = b->nrhs;
     std::vector<ResidentSystem> sys;

@@ -202,6 +202,9 @@ struct fk_context {
     int num_cus = 256;
     bool graphs = true;  // capture PCG iteration chunks in hipGraphs (FEMEKO_HIP_GRAPHS=0 disables)
     bool resident = true;  // solves in one resident launch where the mesh fits (FEMEKO_HIP_RESIDENT=0 disables)
+    // all-reduces of a launch before its waits give up (FEMEKO_HIP_RESIDENT_ROUNDS, for tests of the way back)
+    uint32_t resident_rounds = UINT32_MAX;
+    int32_t resident_skip = 0, resident_pause = 0;  // after a wait that ran out: solves still, and then, without one
     bool one_shot = false;  // destroyed by the call that made it: no copy threads
     std::string err;
     fk::TimingEvents timing;
@@ -383,6 +386,7 @@ inline void values_changed(fk_mesh *m) {
     m->sell64_valid = false;
     m->sell32_valid = false;
 }
+bool resident_allowed(fk_context *c);  // for the solve at hand
 // FP64 PCG in one cooperative launch (resident.hip); false: not for this mesh
 bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, CgState *out);
 void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::vector<int32_t> &ci,

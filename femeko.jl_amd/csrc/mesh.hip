@@ -372,6 +372,9 @@ int fk_context_create(int device, fk_context **out) {
         ctx->graphs = g ? g[0] != '0' : !profiled;
         const char *r = std::getenv("FEMEKO_HIP_RESIDENT");
         ctx->resident = !(r && r[0] == '0');
+        const char *k = std::getenv("FEMEKO_HIP_RESIDENT_ROUNDS");
+        if (k && k[0] != '\0')
+            ctx->resident_rounds = static_cast<uint32_t>(std::strtoul(k, nullptr, 10));
         FK_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
         fk::noalloc_setup(device);
     } catch (const fk::Error &e) {

@@ -81,7 +81,9 @@ __device__ __forceinline__ double fold4(double a, double b, double c, double d) 
 // memory and 12 us: all blocks polling the few group sums wait for each other.
 //
 // Waits are bounded: after kSpinLimit polls (about a second; a co-resident
-// block answers in microseconds) the round fails and the kernel ends.
+// block answers in microseconds) the round fails and the kernel ends. The round
+// with tag 0, which tags counted up from a first one of 1 do not reach, fails
+// at its first poll.
 constexpr int kSpinLimit = 1 << 20;
 constexpr int kMaxResidentBlocks = 256;
 constexpr int kReduceCopies = 8;
@@ -130,7 +132,7 @@ __device__ __forceinline__ bool all_reduce5(double (&v)[5], u64 *__restrict__ li
         u64 a[PER];
 #pragma unroll
         for (int i = 0; i < PER; ++i) a[i] = tag;  // a lane without a word holds the tag over zero
-        int spin = 0;
+        int spin = tag == 0 ? kSpinLimit : 0;
         uint32_t miss;
         do {
 #pragma unroll

@@ -86,6 +86,7 @@ struct ResidentArgs {
     int32_t us;                   // distance of a row's values in u and r64 (right-hand sides side by side)
     double s, target2, thresh64, delta2;
     int32_t G;                    // iterations between two checks of the drop
+    uint32_t first;               // tag of the first exchange; the waits of tag 0 give up
 };
 
 // A copy of v that the compiler takes for a new value: addresses computed from
@@ -186,7 +187,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
     };
     const int32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int32_t h0 = GEN ? A.halo_ptr[i0 / R] : 0, nh = GEN ? A.halo_ptr[i0 / R + 1] - h0 : 0;
-    uint32_t tag = 1;
+    uint32_t tag = A.first;
     if (tid == 0) sh[kReduceShared - 1] = 0.0;
 
     // z = D^-1 r of the own rows goes out
@@ -853,6 +854,7 @@ static bool launch_resident(fk_mesh *m, ResidentArgs<T> &A) {
     const size_t lds = (static_cast<size_t>(elements) + 1 + x_in_lds<T>(RPT, NE < 0) * BLOCK) * sizeof(T);
     if (lds > static_cast<size_t>(kResLdsMax)) return false;
     A.nb = nb;
+    A.first = 0u - m->ctx->resident_rounds;
     // rows past the last, as far as the last block's windows reach, read zero
     const int64_t reach = NE < 0 ? m->nv : static_cast<int64_t>(nb) * R + (NE > 0 ? 0 : m->st_off[m->st_K - 1] + R);
     const int64_t stride = (reach + 63) / 64 * 64;
@@ -1069,15 +1071,31 @@ void build_resident_sell(fk_mesh *m, const std::vector<int32_t> &rp, const std::
     }
 }
 
+bool resident_allowed(fk_context *c) {
+    if (c->timing.enabled || !c->resident) return false;
+    if (c->resident_skip == 0) return true;
+    --c->resident_skip;
+    return false;
+}
+
+// A wait that runs out costs about a second. Another process that keeps the
+// CUs does so for longer than one solve: the solves that follow it, 8 and after
+// every further time-out in a row twice as many up to 1024, run on the three
+// kernels before one is tried again.
+static bool timed_out(fk_context *c, bool yes) {
+    c->resident_pause = yes ? std::min(std::max(2 * c->resident_pause, 8), 1024) : 0;
+    c->resident_skip = c->resident_pause;
+    return yes;
+}
+
 // the copy of the matrix a resident launch can run on, with fresh values
 static bool resident_kind(const fk_mesh *m) {
-    if (m->ctx->timing.enabled || !m->ctx->resident) return false;
     if (m->kind == FK_SPMV_STENCIL) return m->st_K <= kResK;
     return m->kind == FK_SPMV_SELL64 && m->format != FK_SPMV_CSR && m->have_sell && m->res_R > 0;
 }
 
 bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, CgState *out) {
-    if (!resident_kind(m)) return false;
+    if (!resident_kind(m) || !resident_allowed(m->ctx)) return false;
     const bool stencil = m->kind == FK_SPMV_STENCIL;
     PcgWork<double> &w = m->w64;
     ResidentArgs<double> A{};
@@ -1101,7 +1119,7 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
     FK_HIP(hipMemcpyAsync(hs, w.state.get(), sizeof(CgState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
     // a wait ran out (another process's launch); r0 is unchanged
-    if (hs->status == FK_ERR_HIP || hs->timed_out) return false;
+    if (timed_out(m->ctx, hs->status == FK_ERR_HIP || hs->timed_out)) return false;
     *out = *hs;
     return true;
 }
@@ -1112,7 +1130,7 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
 bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double thresh, double delta, int64_t max_iter,
                       int chunk, int64_t *iters, int32_t *nrep, double *rr_out, int *status, bool *started) {
     *started = false;
-    if (!resident_kind(m)) return false;
+    if (!resident_kind(m) || !resident_allowed(m->ctx)) return false;
     const bool stencil = m->kind == FK_SPMV_STENCIL;
     PcgWork<float> &w = m->w32;
     if (!m->ru) {
@@ -1149,7 +1167,7 @@ bool resident_refined(fk_mesh *m, double *u, const double *b, double rr, double 
     FK_HIP(hipMemcpyAsync(hs, w.state.get(), sizeof(CgState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipMemcpyAsync(hr, m->ru.get(), sizeof(RuState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
-    if (hr->status == FK_ERR_HIP) return false;  // a wait ran out (another process's launch)
+    if (timed_out(m->ctx, hr->status == FK_ERR_HIP)) return false;  // a wait ran out (another process's launch)
     *iters = hs->iters;
     *nrep = hr->nrep;
     *rr_out = hr->rr64;
@@ -1257,6 +1275,7 @@ static bool launch_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sy
         A.thresh64 = q.thresh64;
         A.delta2 = delta * delta;
         A.G = chunk;
+        A.first = 0u - ctx->resident_rounds;
         words += reduce_words(A.nb);
         floats += 2 * static_cast<int64_t>(A.stride);
     }
@@ -1303,11 +1322,11 @@ bool resident_batch(ResidentBatch &B, const std::vector<ResidentSystem> &sys, do
     FK_HIP(hipMemcpyAsync(state.data(), B.state.get(), S * sizeof(CgState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipMemcpyAsync(ru.data(), B.ru.get(), S * sizeof(RuState), hipMemcpyDeviceToHost, st));
     FK_HIP(hipStreamSynchronize(st));
-    for (const RuState &r : ru)
-        if (r.status == FK_ERR_HIP) {  // a wait ran out (another process's launch)
-            B.rows = B.launches = 0;
-            return false;
-        }
+    const bool late = std::any_of(ru.begin(), ru.end(), [](const RuState &r) { return r.status == FK_ERR_HIP; });
+    if (timed_out(B.ctx, late)) {  // a wait ran out (another process's launch)
+        B.rows = B.launches = 0;
+        return false;
+    }
     return true;
 }
 
