@@ -15,8 +15,9 @@ remaining error sits in smooth modes that weigh little in the residual).
 
 Reported beside the headline: the plain FP64 GPU solve of the same system
 (speed-up), the classic restarted refinement (FP32 PCG to 1e-5 inside an FP64
-residual-correction loop), the SpMV kernel's achieved bandwidth (back-to-back
-launches between two HIP events on the library stream), and, after the GPU
+residual-correction loop), the solve's achieved bandwidth per iteration where
+it runs in one resident launch, the SpMV kernel's of the three-kernel iteration
+(back-to-back launches between two HIP events on the library stream), and, after the GPU
 part, the oracle on the host cores: its full assembly and Jacobi-PCG solve of
 the same system to the FP64 path's tolerance (the CPU baseline, plus a
 1-thread sample), continued to rtol 1e-13 as the FP64 reference that the
@@ -166,6 +167,29 @@ def _pmc_traffic(args, solver_format):
     if solver_format == "sell64" and vals.get("shape") != args.shape:
         return None
     return float(vals["traffic_bytes_per_launch"])
+
+
+def _resident_roofline(args, K, nv, block_rows, t_iter):
+    """An iteration of a solve on bricks streams the K value columns once (the
+    vectors stay on the chip); its time is the timed solve's over its
+    iterations, residual replacements and launch included."""
+    B = K * 4 * nv
+    achieved = B / t_iter / 1e9
+    r = {"bound": "hbm", "kernel": "k_resident_pcg<float> on bricks, one launch per solve", "achieved": achieved,
+         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": None,
+         "bytes_per_iteration": B, "bytes_basis": "stencil copy: K*4*nv values",
+         "us_per_iteration": t_iter * 1e6, "us_per_iteration_basis": "timed step less assembly, over its iterations"}
+    vals = {}
+    path = os.path.join(ROOT, "profiles", "pmc_resident.txt")
+    if args.n == 160 and args.renumber == "none" and os.path.exists(path):
+        with open(path) as fh:
+            vals = dict(line.strip().split(": ", 1) for line in fh if line.count(": ") == 1)
+    if vals.get("rows_per_block") == str(block_rows):
+        # HBM bytes per iteration from the committed counter profile
+        r["traffic"] = float(vals["traffic_bytes_per_iteration"])
+        r["traffic_GBs"] = r["traffic"] / t_iter / 1e9
+        r["traffic_frac"] = r["traffic_GBs"] / HBM_PEAK_GBS
+    return r
 
 
 def _common(args, metric, value, unit, ms, dtype, config, higher=True):
@@ -566,6 +590,8 @@ def main():
     t_step = (time.perf_counter() - t0) / args.steps
     log(f"f32-refined step {t_step*1e3:.1f} ms, iterations {rep.iterations}, outer {rep.outer}, "
         f"relres {rep.relres:.2e}")
+    layout, block_rows, blocks = dm.solve_launch()
+    log(f"solve launch: {layout}" + (f", {blocks} blocks of {block_rows} rows" if blocks else ""))
     phi32 = dm.potential()
     _H, Hn32, E32 = dm.field(want_H=False, want_Hn=True, want_energy=True)
     # assembly alone
@@ -600,6 +626,8 @@ def main():
     log(f"copy probe: 1 GiB in {copy_ms:.3f} ms, {copy_gbs:.0f} GB/s read+write")
 
     # ---- SpMV kernel timing: HIP events around every SpMV launch of one instrumented solve
+    # (timing keeps the context to the three kernels per iteration, so this is
+    # the solve of meshes that run in no resident launch)
     ctx.set_timing(True)
     dm.assemble()
     t0 = time.perf_counter()
@@ -624,7 +652,7 @@ def main():
         B32 = B_csr
     achieved = B32 / (spmv_us * 1e-6) / 1e9
     log(f"SpMV f32: {spmv_us:.1f} us per launch back to back, {achieved:.0f} GB/s; "
-        f"{spmv_us_in_solve:.1f} us avg over {launches} launches in a solve with events around each")
+        f"{spmv_us_in_solve:.1f} us avg over {launches} launches in a three-kernel solve with events around each")
 
     out = {
         "metric": METRIC,
@@ -667,6 +695,7 @@ def main():
         "fp64": {"ms_per_step": t_step64 * 1e3, "iterations": rep64.iterations, "relres": rep64.relres,
                  "dof_per_s": m.nv / t_step64},
         "speedup_vs_fp64": t_step64 / t_step,
+        "solve_launch": {"layout": layout, "rows_per_block": block_rows, "blocks": blocks},
         "roofline": {
             "bound": "hbm",
             "kernel": {"csr": "k_cg_spmv<float,%d>" % args.lanes,
@@ -709,6 +738,12 @@ def main():
         out["roofline"]["traffic"] = traffic
         out["roofline"]["traffic_GBs"] = traffic / (spmv_us * 1e-6) / 1e9
         out["roofline"]["traffic_frac"] = out["roofline"]["traffic_GBs"] / HBM_PEAK_GBS
+    if layout == "bricks":
+        # the timed step ran in one resident launch: its own roofline, the
+        # product of the three-kernel solve beside it
+        out["spmv"] = out["roofline"]
+        out["roofline"] = _resident_roofline(args, len(stencil_offsets), m.nv, block_rows,
+                                             (t_step - t_asm) / max(rep.iterations, 1))
     dm.close()
     if not args.no_cpu:
         nthreads = min(16, os.cpu_count() or 1)

@@ -1896,12 +1896,18 @@ static int solve_f32_replace(fk_mesh *m, double *u, const double *b, double rtol
     *rr_out = rr;
     if (rr < thresh) return FK_OK;
     const int G = nv > 200000 ? 32 : 16;
+    const char *tr = std::getenv("FEMEKO_HIP_TRACE");
+    const bool trace = tr && tr[0] == '1';
     sync_solver_values<float>(m);
     if (std::isfinite(rr)) {
         int status = FK_OK;
         bool started = false;
-        if (resident_refined(m, u, b, rr, thresh, delta, max_iter, G, iters, nrep, rr_out, &status, &started))
+        if (resident_refined(m, u, b, rr, thresh, delta, max_iter, G, iters, nrep, rr_out, &status, &started)) {
+            if (trace)
+                std::fprintf(stderr, "[fk trace] resident launch: iterations %lld replacements %d restarts %d rr64 %.3e\n",
+                             static_cast<long long>(*iters), *nrep, m->hru.ptr->restarts, *rr_out);
             return status;
+        }
         if (started) rr = neg_residual(m, u, m->r64.get(), b);
     }
     three_kernels(m);
@@ -1927,8 +1933,6 @@ static int solve_f32_replace(fk_mesh *m, double *u, const double *b, double rtol
     init.delta2 = delta * delta;
     FK_HIP(hipMemcpyAsync(m->ru.get(), &init, sizeof(RuState), hipMemcpyHostToDevice, st));
     m->part_misc.ensure(nb);
-    const char *tr = std::getenv("FEMEKO_HIP_TRACE");
-    const bool trace = tr && tr[0] == '1';
     const bool timed = m->ctx->timing.enabled;
     RuState *hr = m->hru.ptr;
     CgState *hs = m->hstate.ptr;

@@ -429,9 +429,12 @@ int fk_batch_set_launch(fk_batch *batch, int32_t lanes, int32_t block);
 int fk_batch_launch(fk_batch *batch, int32_t *lanes, int32_t *block, int32_t *spmm_block, int32_t *spmm_rows);
 
 /* ---- instrumentation -------------------------------------------------------
- * Average device time of the sparse matrix-vector kernel over the last solve
- * (HIP events on the context stream around each launch), when enabled with
- * fk_set_timing(ctx, 1). Returns launches and total milliseconds. */
+ * Device time of the sparse matrix-vector kernel over the solves since timing
+ * was enabled with fk_set_timing(ctx, 1) (HIP events on the context stream
+ * around each launch): launches and total milliseconds. A context with timing
+ * enabled solves on the three kernels per iteration, one of which is that
+ * product; otherwise a mesh that fits is solved in one resident launch
+ * (fk_solve_launch), to which these figures do not apply. */
 int fk_set_timing(fk_context *ctx, int32_t enable);
 int fk_spmv_timing(fk_context *ctx, int64_t *launches, double *total_ms);
 /* Streaming-bandwidth probe: copy `bytes` (a multiple of 16 is used) between

@@ -152,6 +152,16 @@ def test_three_kernels_in_graphs(contexts, n, scattered, precision):
         timed.close()
 
 
+def test_trace(contexts, capfd, monkeypatch):
+    """FEMEKO_HIP_TRACE=1 reports a refined solve on either path."""
+    monkeypatch.setenv("FEMEKO_HIP_TRACE", "1")
+    pr = W.linear(20)
+    for ctx, text in zip(contexts, ("[fk trace] resident launch: iterations {} replacements {} ",
+                                    "[fk trace] replacements {1} ")):
+        _, rep, _, _ = _solve(ctx, pr.mesh, pr.mu, pr.mask, pr.g, "f32", 1e-10)
+        assert text.format(rep.iterations, rep.outer) in capfd.readouterr().err
+
+
 @pytest.mark.parametrize("boxes,nrhs,rows", [([(1, 1, 1)], 1, 512), ([(20, 20, 20)] * 3 + [(3, 4, 5)], 2, 512),
                                              ([(28, 28, 28)] * 7 + [(15, 15, 31), (2, 1, 3)], 3, 2048)])
 def test_batch(contexts, boxes, nrhs, rows):
