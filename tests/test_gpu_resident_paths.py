@@ -100,6 +100,48 @@ def test_scattered(contexts, precision, n, layout, rows):
     _check(contexts, pr.mesh, pr.mu, pr.mask, pr.g, precision, (layout, rows))
 
 
+def _split(pr, extra):
+    """The problem with `extra` elements at each of a few nodes split at their
+    centroid: rows of 14 + extra entries there."""
+    t = np.asarray(pr.mesh.t, dtype=np.int64) - 1
+    used = np.zeros(pr.mesh.nv, bool)
+    pick = []
+    for node in np.random.default_rng(extra).permutation(pr.mesh.nv):
+        around = np.flatnonzero((t == node).any(axis=0))
+        if around.size == 24 and not used[t[:, around]].any():
+            used[t[:, around]] = True
+            pick.extend(around[:extra])
+        if len(pick) >= 3 * extra:
+            break
+    pick = np.array(pick)
+    corner = t[:, pick]
+    new = pr.mesh.nv + np.arange(pick.size)
+    p = np.concatenate([pr.mesh.p, pr.mesh.p[:, corner].mean(axis=1)], axis=1)
+    parts = [np.delete(t, pick, axis=1)]
+    for k in range(4):
+        c = corner.copy()
+        c[k] = new
+        parts.append(c)
+    mu = np.concatenate([np.delete(pr.mu, pick)] + [pr.mu[pick]] * 4)
+    t = np.concatenate(parts, axis=1)
+    order = np.random.default_rng(1).permutation(p.shape[1])
+    inv = np.argsort(order)
+    p, t = np.asfortranarray(p[:, order]), np.asfortranarray((inv[t] + 1).astype(np.int32))
+    fill = np.zeros(pick.size)
+    mask = np.concatenate([pr.mask, fill.astype(np.uint8)])[order]
+    return MESH(p=p, t=t, VE=element_volumes(p, t)), mu, mask, np.concatenate([pr.g, fill])[order]
+
+
+# rows of up to 18 (20 with padding) and 26 entries
+@pytest.mark.parametrize("precision,n,extra,layout,rows", [
+    ("f64", 20, 4, "sell", 512), ("f64", 50, 4, "sell", 1024), ("f64", 64, 4, *KERNELS), ("f64", 20, 12, "sell", 512),
+    ("f64", 50, 12, *KERNELS), ("f32", 20, 4, "sell", 512), ("f32", 50, 4, "sell", 1024), ("f32", 64, 4, "sell", 1536),
+    ("f32", 79, 4, "sell", 2048), ("f32", 20, 12, "sell", 512), ("f32", 50, 12, "sell", 1024), ("f32", 64, 12, *KERNELS)])
+def test_longer_rows(contexts, precision, n, extra, layout, rows):
+    mesh, mu, mask, g = _split(W.linear(n), extra)
+    _check(contexts, mesh, mu, mask, g, precision, (layout, rows))
+
+
 @pytest.mark.parametrize("precision,dims,layout,rows", [
     ("f64", (30, 30, 600), "bricks", 2560), ("f64", (400, 400, 3), *KERNELS), ("f64", (230, 47, 55), "windows", 2560),
     ("f32", (400, 400, 3), "windows", 3072), ("f32", (230, 47, 55), "bricks", 5120)])
