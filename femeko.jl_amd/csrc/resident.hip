@@ -105,9 +105,15 @@ __device__ __forceinline__ int32_t window_lds(Args &A, int32_t R, int32_t e) {
 }
 template <typename Args>
 __device__ __forceinline__ int32_t window_row(Args &A, int32_t i0, int32_t li) {
-    int32_t d = A.wrow[0];
+    // FP64 selects values: the compiler else selects the address and loads it,
+    // a trip to memory before every element's w, one after another at four rows
+    // per thread
+    const auto at = [&](int k) {
+        return sizeof(*A.val) == 8 ? __builtin_amdgcn_readfirstlane(A.wrow[k]) : A.wrow[k];
+    };
+    int32_t d = at(0);
 #pragma unroll
-    for (int k = 1; k < kResWindows; ++k) d = li >= A.wbeg[k] ? A.wrow[k] : d;
+    for (int k = 1; k < kResWindows; ++k) d = li >= A.wbeg[k] ? at(k) : d;
     return li < A.wbeg[kResWindows] ? i0 + li + d : -1;
 }
 
@@ -132,6 +138,7 @@ __device__ __forceinline__ double reciprocal(double v) {
     return v != 0.0 ? fma(y, fma(-v, y, 1.0), y) : 0.0;
 }
 
+constexpr int64_t kClosing = int64_t(1) << 62;  // added to the iterations in the last round; past any limit
 constexpr int kResRestarts = 32;  // direction restarts before the FP32 recursion gives up
 
 // RPT rows per thread, the values of the first NK of them in registers (the
@@ -158,6 +165,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
     extern __shared__ char lds_raw[];
     T *win = reinterpret_cast<T *>(lds_raw);
     __shared__ double sh[kReduceShared];
+    [[maybe_unused]] __shared__ double before;  // thread 0: ||r||^2 before the step on the way out
     constexpr int K = kResK, R = BLOCK * RPT;
     constexpr bool GEN = NE > 0, BRICK = NE < 0;
     constexpr int TP = BRICK ? -NE : 1, BZ = RPT / TP;  // runs of BLOCK rows in a plane of a brick, planes
@@ -319,14 +327,13 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
             for (int j = 0; j < NK; ++j) load_row(own_row(j, tl), v[j]);
         }
         [[maybe_unused]] bool moved = false;  // an iteration done in this run
-        [[maybe_unused]] int closing = 0;     // FP64: the last round, with p = z
-        [[maybe_unused]] int step = 0;        // and the step on the way out
+        // FP64, converged: 1 the round of q = A z, 2 that of the residual after the step
+        [[maybe_unused]] int closing = 0;
+        [[maybe_unused]] bool undo = false;
+        constexpr T third = T(1.0 / 3.0);
         [[maybe_unused]] int act = 0;         // why it ended: 1 replace r, 2 drop x and restart
         while (true) {
             ++tag;
-            // one loop body for both kinds of round: a copy for the last one costs
-            // every FP64 shape 7 to 40 registers
-            const bool last = !REFINE && __builtin_amdgcn_readfirstlane(fresh(closing)) != 0;
             // q = A p in difference form; w = D^-1 q
 #pragma unroll
             for (int k = 0; k < 5; ++k) s[k] = 0.0;
@@ -357,9 +364,9 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                     const double zd = static_cast<double>(z[j]), qd = static_cast<double>(q);
                     const double rd = static_cast<double>(reciprocal(d[j]) * z[j]);
                     // past a run pj is any LDS word
-                    s[0] += (last ? rd : static_cast<double>(d[j] != T(0) ? pj : T(0))) * qd;
+                    s[0] += static_cast<double>(d[j] != T(0) ? pj : T(0)) * qd;
                     s[1] += rd * zd;
-                    s[2] += qd * (last ? qd : zd);
+                    s[2] += qd * zd;
                     s[3] += qd * static_cast<double>(w[j]);
                     s[4] += rd * rd;
                     __builtin_amdgcn_sched_barrier(0);
@@ -413,9 +420,9 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                 rows.store(tag, row, w[j]);  // 0 past the last row
                 const double zd = static_cast<double>(z[j]), qd = static_cast<double>(q);
                 const double rd = static_cast<double>(g[j] * z[j]);
-                s[0] += (last ? rd : static_cast<double>(p[j])) * qd;
+                s[0] += static_cast<double>(p[j]) * qd;
                 s[1] += rd * zd;
-                s[2] += qd * (last ? qd : zd);
+                s[2] += qd * zd;
                 s[3] += qd * static_cast<double>(w[j]);
                 s[4] += rd * rd;
                 __builtin_amdgcn_sched_barrier(0);
@@ -460,18 +467,36 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                        : !(pq > 0.0) || !isfinite(pq)          ? FK_ERR_SINGULAR  // not positive definite on the space
                                                                : -1;
                 code = __builtin_amdgcn_readfirstlane(code);
-                if (last) {  // q = A z: the sums hold r.q and q.q
-                    const double after = rr - (2.0 / 3.0) * pq + s[2] / 9.0;
-                    code = alive ? FK_OK : FK_ERR_HIP;
-                    step = __builtin_amdgcn_readfirstlane(after < thresh);
-                    if (step) rr = fmax(after, 0.0);
-                    break;
-                }
-                // a converged recursion that has moved x goes one round more with p = z
-                closing = __builtin_amdgcn_readfirstlane(code == FK_OK && it > 0 && pq > 0.0 && isfinite(pq) &&
-                                                         isfinite(s[3]));
-                if (code >= 0 && !closing) break;
-                if (closing) {
+                if (code >= 0) {
+                    // a converged recursion that has moved x goes two rounds more. One
+                    // loop body for all rounds (fresh): copies of it for the last two
+                    // cost every FP64 shape 7 to 40 registers
+                    const int phase = __builtin_amdgcn_readfirstlane(fresh(closing));
+                    if (!alive) break;
+                    if (phase == 2) {  // r after the step
+                        it -= kClosing;
+                        undo = !(rr < thresh);
+                        if (undo && tid == 0) rr = before;
+                        code = FK_OK;
+                        break;
+                    }
+                    if (phase == 1) {  // p = z, w = D^-1 A z: the step; p stays, to take it back
+#pragma unroll
+                        for (int j = 0; j < RPT; ++j) {
+                            if constexpr (BRICK) {
+                                if ((j % TP) * BLOCK + ft < blen) xj(j, ft) += third * win[own_lds(j, ft)];
+                            } else {
+                                xj(j, ft) += third * p[j];
+                            }
+                            z[j] -= third * w[j];
+                        }
+                        if (tid == 0) before = rr;
+                        it += kClosing;  // the next round ends here whatever r is
+                        closing = 2;
+                        continue;
+                    }
+                    if (code != FK_OK || it == 0 || !(pq > 0.0) || !isfinite(pq) || !isfinite(s[3])) break;
+                    closing = 1;
                     alpha = beta = T(0);
                     --it;
                 }
@@ -508,7 +533,7 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
                 const int32_t row = own_row(j, tid);
-                // One Jacobi step of 1/3 on the way out. The largest eigenvalues
+                // One Jacobi step of 1/3 was done on the way out. The largest eigenvalues
                 // of D^-1 A are those of slivers, 2 to 4 (4: flat, four nodes; the
                 // scaled matrix of an element with parallel gradients has rank one
                 // and trace 4). Rounding brings their modes back late in the
@@ -518,11 +543,20 @@ __device__ __forceinline__ void resident_solve(Args &A, const int me, const int3
                 // 1e-10 over its rms, 8 jittered meshes of 63^3 cells (jitter 0.2
                 // to 0.26): 2.4e-9 to 1.6e-7 with the step, 1.9e-9 to 3.1e-7 after
                 // the three kernels. ||r|| itself mostly falls by 0.7 but may rise
-                // (1.13 times on a graded Delaunay mesh), so the closing round
-                // measures it and the step is taken where it stays below the
-                // tolerance; the residual reported is that of the x returned.
-                const T xr = xj(j, tid);
-                if (row < n) A.x[row] = step ? xr + T(1.0 / 3.0) * z[j] : xr;
+                // (1.25 times on a graded Delaunay mesh), so a round of its own
+                // measures it after the step, which is taken back where it does
+                // not stay below the tolerance; the residual reported is that of
+                // the x returned. Weighing the sums of one round instead (r.q and
+                // q.q) cost two selects a row in all rounds, 1% of a solve.
+                if (row < n) {
+                    const T xr = xj(j, tid);
+                    T pj;
+                    if constexpr (BRICK)
+                        pj = win[own_lds(j, tid)];
+                    else
+                        pj = p[j];
+                    A.x[row] = undo ? xr - third * pj : xr;
+                }
             }
             break;
         } else {
@@ -1109,7 +1143,7 @@ bool resident_pcg_f64(fk_mesh *m, double rtol, int64_t max_iter, double bb_ref, 
     A.K = m->st_K;
     A.bb_ref = bb_ref;
     A.rtol = rtol;
-    A.max_iter = max_iter;
+    A.max_iter = std::min(max_iter, kClosing / 2);
     // one resident launch of this process at a time on the device: the blocks
     // of two would take each other's CUs and wait for blocks not yet started
     const std::lock_guard<std::mutex> alone(resident_mutex(m->ctx->device));
