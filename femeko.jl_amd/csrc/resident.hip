@@ -937,18 +937,18 @@ static int64_t rows_per_block(const fk_mesh *m) {
 // wastes 1 to 20% of them. Measured per iteration (us; in
 // brackets the windows or, for FP64 n > 100 and FP32 n > 126, the three kernels),
 // Kuhn meshes of n cells per side:
-//   FP64  n = 80  8.8 (10.9)   n = 90 11.6 (14.1)   n = 95 11.7 (18.5)   n = 100 13.7 (22.2)
-//         n = 105 16 (41.5)    n = 118 21 (52.7)    n = 125 24 (60.0)    n = 130 35 (67.5)
-//   FP32  n = 80  7.5 (8.7)    n = 95 9 (11.5)      n = 100 10.6 (13.5)  n = 118 14.0 (20.5)
-//         n = 126 16.3 (28.8)  n = 140 21.6 (45.6)  n = 150 25 (53.8)    n = 160 29.0 (61.8)
+//   FP64  n = 80  8.9 (10.9)   n = 90 11.0 (14.1)   n = 95 11.7 (18.5)   n = 100 13.9 (22.2)
+//         n = 105 15.9 (41.5)  n = 118 19.7 (52.7)  n = 125 25.9 (60.0)  n = 130 33.2 (67.5)
+//   FP32  n = 80  7.8 (8.7)    n = 95 9.0 (11.5)    n = 100 10.6 (13.5)  n = 118 14.5 (20.5)
+//         n = 126 16.1 (28.8)  n = 140 22.2 (45.6)  n = 150 25.3 (53.8)  n = 160 29.7 (61.8)
 // More rows in flight (2 or 3 per thread) were no faster at any size: n = 160
 // 40.0 us with 3, where they spill, n = 115 14.9 with 2 or 3. What bounds the
-// larger ones is the value stream from the MALL: of 29.0 us at n = 160, 12.3 go
+// larger ones is the value stream from the MALL: of 29 us at n = 160, 12.3 go
 // away when the values (7 columns, 117 MB) are not loaded and 3.0 without the
 // exchange; 3.2 are the residual replacements, one in 63 iterations.
 //
 // Up to four rows per thread the windows, which keep the values in registers,
-// are faster: FP64 n = 76 7.1 us against 7.8, n = 70 6.3 against 7.9.
+// are faster: FP64 n = 76 6.8 us against 7.8, n = 70 6.0 against 7.9.
 constexpr int64_t kBrickRows = 2048;
 
 template <typename T, int BZ, int TP>
@@ -974,13 +974,14 @@ static bool launch_bricks(fk_mesh *m, ResidentArgs<float> &A) {
 // for all their matrix values in registers (NK = RPT) and shorten every step
 // between two exchanges. Measured per iteration (us; three-kernel iteration in
 // brackets), Kuhn meshes of n cells per side:
-//   n = 20  512 x 1   3.9 (14.7)     n = 40  512 x 1   4.2 (15.9)
-//   n = 63  512 x 2   4.8 (21.5)     n = 70  512 x 3   6.4 (23.7)
-//   n = 79  512 x 4   7.6 (26.9)     n = 85  512 x 5  11.3 (29.4)
-//   n = 90  512 x 6  14.5 (31.5)     n = 95  512 x 7  17.8 (34)
-//   n = 100 512 x 8  21.8 (36.8)
-// The last four shapes serve stencils that are cut into no bricks.
-// One shape up costs: n = 63 on 512 x 3 5.8, n = 79 on 512 x 5 10.9, n = 85 on
+//   n = 20  512 x 1   3.1 (14.7)     n = 40  512 x 1   3.6 (15.9)
+//   n = 63  512 x 2   4.5 (21.5)     n = 70  512 x 3   6.0 (23.7)
+//   n = 79  512 x 4   7.3 (26.9)     n = 84  512 x 5   8.8 (29.4)
+//   n = 90  512 x 6  13.4 (31.5)     n = 95  512 x 7  16.1 (34)
+//   n = 99  512 x 8  18.5 (36.8)
+// The last four shapes serve stencils that are cut into no bricks (measured on
+// boxes cut along their other diagonal).
+// One shape up costs (when the shape taken was at 4.8, 7.6 and 11.3): n = 63 on 512 x 3 5.8, n = 79 on 512 x 5 10.9, n = 85 on
 // 512 x 6 13.6. More rows than 256 blocks of 4096 keep the three-kernel
 // iteration: the windows of more rows per block exceed the LDS.
 static bool launch_by_rows(fk_mesh *m, ResidentArgs<double> &A) {
@@ -999,11 +1000,13 @@ static bool launch_by_rows(fk_mesh *m, ResidentArgs<double> &A) {
 
 // The same for the FP32 recursion with residual replacement, half the
 // registers and LDS per row. Measured as above, replacements included:
-//   n = 20  512 x 1   4.2 (14.5)     n = 48  512 x 1   5.1 (15.7)
-//   n = 63  512 x 2   5.2 (19.0)     n = 75  512 x 4   6.9 (20.7)
-//   n = 90 1024 x 3   9.7 (22.8)     n = 100 512 x 8  13.7 (25.2)
-//   n = 115 512 x 12 20   (31)       n = 126 512 x 16 28.1 (35.6)
-// The last four shapes serve stencils that are cut into no bricks.
+//   n = 20  512 x 1   3.8 (14.5)     n = 48  512 x 1   4.9 (15.7)
+//   n = 63  512 x 2   5.0 (19.0)     n = 75  512 x 4   6.4 (20.7)
+//   n = 85 1024 x 3   9.4 (22.8)     n = 98  512 x 8  12.9 (25.2)
+//   n = 110 512 x 12 19.9 (31)       n = 125 512 x 16 27.5 (35.6)
+// The last four shapes serve stencils that are cut into no bricks. Below 400k
+// rows an iteration takes longer than in FP64 (the replacements); who asks for
+// FP32 there gets it.
 static bool launch_by_rows(fk_mesh *m, ResidentArgs<float> &A) {
     const int64_t per = rows_per_block(m);
     if (per > kBrickRows && launch_bricks(m, A)) return true;
@@ -1027,12 +1030,14 @@ static int sell_rows_per_block(const fk_mesh *m, int width) {
 }
 
 // By the longest row (up to 16 entries: a numbering of a structured mesh; 20:
-// the same with slices padded to a common offset set; 32: Delaunay meshes) and
-// the rows per block. The values, LDS indices and halo of more rows do not fit
-// the registers. Measured per iteration (us; three-kernel iteration in
+// the same with slices padded to a common offset set; 32: Delaunay meshes of
+// some hundred nodes) and the rows per block. One longer row keeps the whole
+// mesh on the three kernels: so do Delaunay meshes of 4k nodes and more, where
+// one row in 500 has 33 to 65. The values, LDS indices and halo of more rows do
+// not fit the registers. Measured per iteration (us; three-kernel iteration in
 // brackets), randomly numbered Kuhn meshes:
-//   FP64  n = 20 3.4 (14.0)  n = 41 3.7 (15.9)  n = 55 4.7 (24.4)  n = 70 7.7 (29.6)
-//   FP32  n = 20 4.3 (15.3)  n = 41 5.0 (17.4)  n = 55 6.6 (21.2)  n = 70 6.7 (24.8)
+//   FP64  n = 20 2.8 (14.0)  n = 41 3.4 (15.9)  n = 55 4.5 (24.4)  n = 70 7.5 (29.6)
+//   FP32  n = 20 3.8 (15.3)  n = 41 4.7 (17.4)  n = 55 6.4 (21.2)  n = 70 6.5 (24.8)
 static bool launch_sell(fk_mesh *m, ResidentArgs<double> &A) {
     const int w = m->res_width;
     switch (m->res_R) {
